@@ -34,6 +34,16 @@ __device__ __forceinline__ uint16_t float_to_bf16(float v) {
   return (uint16_t)((x + 0x7fffu + ((x >> 16) & 1u)) >> 16);
 }
 
+// Byte offset of value k of row r (0..15) of block b in a 1 KiB tile of the
+// 16-row Q8_1 layout (16 rows x two blocks, b even and odd):
+// [lane quarter][row][block parity][8 values].  Lane 16 q + r of a wave
+// reads 16 B, its MFMA operand of both blocks; the quarters take the values
+// in the order 0, 2, 1, 3 of their eights, which is what two lane swaps
+// make of a weight operand read 16 B at a time (q8_gemm16.hip).
+__device__ __forceinline__ int32_t tile16_offset(int r, int b, int k) {
+  return ((k >> 3 & 1) * 2 + (k >> 4)) * 256 + r * 16 + (b & 1) * 8 + (k & 7);
+}
+
 // RN(1 / s) for s in [2^-125, 2^126]: v_rcp_f32 plus one Newton step with
 // FMA is exact there (checked exhaustively on gfx950 by the device
 // self-test).  Outside that range -- where 1/s is subnormal or overflows --

@@ -137,6 +137,36 @@ struct GemmLaunch {
 
 hipError_t launch_gemm(const GemmLaunch &l, hipStream_t s);
 
+// The GEMM on 16 x 16 tiles (q8_gemm16.hip): the same results for few rows,
+// one launch over up to kMaxGroup weights that share the input rows.  The
+// weights and the tiled rows must each be below 4 GiB.
+struct Gemm16Launch {
+  const int8_t *qa = nullptr;  // Q8_1 input, 16-row tiles (launch_quantize_tiled)
+  const float *sa = nullptr;
+  int64_t m = 0;
+  int64_t cols = 0;            // K
+  bool fma = true;
+  bool y_bf16 = false;
+  const void *add = nullptr;   // residual [m, ldr] of y's element type
+  int64_t ldr = 0;
+  struct Weight {
+    const uint8_t *w = nullptr;
+    const uint8_t *up = nullptr;  // non-null (one weight, no add): the SwiGLU
+                                  // silu(x w^T) * (x up^T)
+    void *y = nullptr;
+    int64_t ldy = 0;
+    int64_t rows = 0;          // N
+    int activation = 0;
+  } w[kMaxGroup];
+  int count = 0;
+};
+hipError_t launch_gemm16(const Gemm16Launch &l, hipStream_t s);
+// Whether m rows go to launch_gemm16, for `count` weights [rows[i] x cols] in
+// one launch (dual: one SwiGLU pair), rather than to launch_gemm for each.
+// split_k: launch_gemm could split K.
+bool gemm16_takes(int64_t m, const int64_t *rows, int count, int64_t cols, bool dual,
+                  bool split_k);
+
 // K splits for a multi-row linear of [m x cols] by [rows x cols] when
 // splitting is allowed: `forced` > 0 (clamped to the pass count), else the
 // count measured fastest for the shape class (tiles x splits within one
@@ -144,19 +174,24 @@ hipError_t launch_gemm(const GemmLaunch &l, hipStream_t s);
 // cover the CUs).
 int32_t gemm_splits_for(int64_t m, int64_t rows, int64_t cols, int32_t forced);
 
-// Q8_1 activations in the GEMM's tiled layout: the 32 rows x 32 values of
-// row tile t and block b are 1 KiB at (t * blocks_pad + b) * 1024 (row r at
-// r * 32), their scales 32 floats at (t * blocks_pad + b) * 32.  Rows past m
-// in the last tile and blocks past the row's are written as zeros.
+// Q8_1 activations in a GEMM's tiled layout.  launch_gemm's: the 32 rows x
+// 32 values of row tile t and block b are 1 KiB at (t * blocks_pad + b) *
+// 1024 (row r at r * 32), their scales 32 floats at (t * blocks_pad + b) *
+// 32.  launch_gemm16's (t16): the 16 rows of row tile t and blocks b, b + 1
+// (b even) are 1 KiB at (t * blocks_pad / 2 + b / 2) * 1024 in the order of
+// tile16_offset, their scales 16 + 16 floats at 32 times that tile index.
+// Rows past m in the last tile and blocks past the row's are written as
+// zeros.
 hipError_t launch_quantize_tiled(const void *x, bool x_bf16, int64_t m,
                                  int64_t ldx, int64_t cols, int8_t *qa,
-                                 float *sa, int64_t blocks_pad, hipStream_t s);
+                                 float *sa, int64_t blocks_pad, bool t16,
+                                 hipStream_t s);
 
 // RMSNorm of m rows of width h (h % 32 == 0) with weight w [h]: y = (x *
 // rstd) * (w or w + 1), each row's sum of squares serial in index order.
 // x and y share their type (f32 or bf16); w is f32 or bf16.  qmode 1 also
-// writes y's Q8_1 in the dense layout (row r at r * blocks_pad * 32, scales
-// at r * blocks_pad), qmode 2 in the tiled layout of launch_quantize_tiled.
+// writes y's Q8_1 in the 16-row layout of launch_quantize_tiled, qmode 2 in
+// its 32-row layout.
 // spec_skew (tests only; 0 otherwise) offsets the predicted partial sums of
 // rows of up to 12288 values, whose serial sum is evaluated speculatively,
 // by that many f32 steps, so that the exact fallbacks decide the results;

@@ -250,13 +250,13 @@ __global__ void quantize_kernel(const void *__restrict__ x, int x_bf16,
   }
 }
 
-// Q8_1 into the GEMM's tiled layout: one wave per 32-row x 1-block tile
-// (tile index rt * blocks_pad + b), in four steps of 8 rows: lane l takes
-// values 4(l%8) .. +3 of row 32rt + 8c + l/8, so each step reads 8 rows of
-// 128 B and writes 256 contiguous bytes of the tile.  quantize_block8 does
-// the arithmetic, so the bits match the row kernel.  Rows past m and blocks
-// past `blocks` are written as zeros.
-template <bool XB, bool AL>
+// Q8_1 into a GEMM's tiled layout, one wave per 1 KiB tile: 32 rows x one
+// block (tile rt * blocks_pad + b), or with T16 16 rows x two blocks (tile
+// rt * blocks_pad / 2 + b / 2, tile16_offset), in four steps of eight rows of
+// one block: lane l takes values 4(l%8) .. +3 of its row, so each step reads
+// eight 128 B runs.  quantize_block8 does the arithmetic, so the bits match
+// the row kernel.  Rows past m and blocks past `blocks` are written as zeros.
+template <bool XB, bool AL, bool T16>
 __global__ __launch_bounds__(256) void quantize_tiles_kernel(
     const void *__restrict__ x, int64_t m, int64_t ldx, int32_t blocks,
     int32_t blocks_pad, int64_t tiles, int8_t *__restrict__ qa,
@@ -264,31 +264,37 @@ __global__ __launch_bounds__(256) void quantize_tiles_kernel(
   const int lane = threadIdx.x & 63;
   const int64_t tile = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (tile >= tiles) return;  // uniform per wave
-  const int32_t rt = (int32_t)(tile / blocks_pad);
-  const int32_t b = (int32_t)(tile - (int64_t)rt * blocks_pad);
+  const int32_t per_row = T16 ? blocks_pad / 2 : blocks_pad;
+  const int32_t rt = (int32_t)(tile / per_row);
+  const int32_t b0 = (int32_t)(tile - (int64_t)rt * per_row) * (T16 ? 2 : 1);
   const int rr = lane >> 3, p = lane & 7;
+  // step c's row within the tile and its block
+  auto row_of = [&](int c) { return T16 ? 8 * (c >> 1) + rr : 8 * c + rr; };
+  auto block_of = [&](int c) { return T16 ? b0 + (c & 1) : b0; };
   // The four loads go out unconditionally (rows past m and padded blocks
   // read a clamped address) and are zeroed only once all are in flight.
-  const int32_t bc = b < blocks ? b : blocks - 1;
   float4 v[4];
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
-    const int64_t row = (int64_t)rt * 32 + 8 * c + rr;
+    const int64_t row = (int64_t)rt * (T16 ? 16 : 32) + row_of(c);
     const int64_t rc = row < m ? row : m - 1;
+    const int32_t bc = block_of(c) < blocks ? block_of(c) : blocks - 1;
     v[c] = load_act4_t<XB, AL>(x, rc * ldx + (int64_t)bc * kBlock + 4 * p);
   }
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
-    const int64_t row = (int64_t)rt * 32 + 8 * c + rr;
-    if (!(row < m && b < blocks)) v[c] = make_float4(0.f, 0.f, 0.f, 0.f);
+    const int64_t row = (int64_t)rt * (T16 ? 16 : 32) + row_of(c);
+    if (!(row < m && block_of(c) < blocks)) v[c] = make_float4(0.f, 0.f, 0.f, 0.f);
   }
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
     int32_t q;
     float s;
     quantize_block8(v[c], true, &q, &s);
-    *(int32_t *)(qa + tile * 1024 + (8 * c + rr) * kBlock + 4 * p) = q;
-    if (p == 0) sa[tile * 32 + 8 * c + rr] = s;
+    const int r = row_of(c);
+    const int32_t off = T16 ? tile16_offset(r, c & 1, 4 * p) : r * kBlock + 4 * p;
+    *(int32_t *)(qa + tile * 1024 + off) = q;
+    if (p == 0) sa[tile * 32 + (T16 ? (c & 1) * 16 : 0) + r] = s;
   }
 }
 
@@ -308,7 +314,7 @@ __global__ __launch_bounds__(256) void quantize_tiles_kernel(
 // chunk of the workgroup's rows and store its squares in the other LDS
 // buffer meanwhile.  Then all waves write y and, with QMODE, its Q8_1 (the
 // quantizer's arithmetic, quantize_block8, on the values as stored): QMODE
-// 1 the dense [m][blocks_pad * 32] layout, QMODE 2 the GEMM's tiled layout
+// 1 the 16-row tiled layout of launch_quantize_tiled, QMODE 2 the 32-row one
 // (blocks past H written as zeros).  Rows past m in the last tile are left
 // unwritten, unlike launch_quantize_tiled, which zeroes them: they hold
 // whatever the workspace held before.  That is harmless only because every
@@ -467,8 +473,9 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(
       quantize_block8(v, valid, &q, &sc);
       if (live) {
         if constexpr (QMODE == 1) {
-          *(int32_t *)(qa + row * ((int64_t)blocks_pad * kBlock) + b * kBlock + 4 * p) = q;
-          if (p == 0) sa[row * blocks_pad + b] = sc;
+          const int64_t tile = (row >> 4) * (blocks_pad / 2) + (b >> 1);
+          *(int32_t *)(qa + tile * 1024 + tile16_offset((int)(row & 15), b, 4 * p)) = q;
+          if (p == 0) sa[tile * 32 + (b & 1) * 16 + (row & 15)] = sc;
         } else {
           const int64_t tile = (row >> 5) * blocks_pad + b;
           *(int32_t *)(qa + tile * 1024 + (row & 31) * kBlock + 4 * p) = q;
@@ -780,8 +787,9 @@ __global__ __launch_bounds__(kSpecThreads) void rmsnorm_spec_kernel(
       float sc;
       quantize_block8(v, true, &qv, &sc);
       if constexpr (QMODE == 1) {
-        *(int32_t *)(qa + row * ((int64_t)blocks_pad * kBlock) + b * kBlock + 4 * p) = qv;
-        if (p == 0) sa[row * blocks_pad + b] = sc;
+        const int64_t tile = (row >> 4) * (blocks_pad / 2) + (b >> 1);
+        *(int32_t *)(qa + tile * 1024 + tile16_offset((int)(row & 15), b, 4 * p)) = qv;
+        if (p == 0) sa[tile * 32 + (b & 1) * 16 + (row & 15)] = sc;
       } else {
         const int64_t tile = (row >> 5) * blocks_pad + b;
         *(int32_t *)(qa + tile * 1024 + (row & 31) * kBlock + 4 * p) = qv;
@@ -793,8 +801,9 @@ __global__ __launch_bounds__(kSpecThreads) void rmsnorm_spec_kernel(
     // blocks past H up to blocks_pad: zeros, as the quantizer gives them
     for (int b = blocks + t / 8; b < blocks_pad; b += kSpecThreads / 8) {
       if constexpr (QMODE == 1) {
-        *(int32_t *)(qa + row * ((int64_t)blocks_pad * kBlock) + b * kBlock + 4 * p) = 0;
-        if (p == 0) sa[row * blocks_pad + b] = 0.0f;
+        const int64_t tile = (row >> 4) * (blocks_pad / 2) + (b >> 1);
+        *(int32_t *)(qa + tile * 1024 + tile16_offset((int)(row & 15), b, 4 * p)) = 0;
+        if (p == 0) sa[tile * 32 + (b & 1) * 16 + (row & 15)] = 0.0f;
       } else {
         const int64_t tile = (row >> 5) * blocks_pad + b;
         *(int32_t *)(qa + tile * 1024 + (row & 31) * kBlock + 4 * p) = 0;
@@ -1160,27 +1169,32 @@ hipError_t launch_quantize(const void *x, bool x_bf16, int64_t m, int64_t ldx,
   return hipGetLastError();
 }
 
+template <bool XB, bool AL>
+static void launch_quantize_tiles(const void *x, int64_t m, int64_t ldx, int64_t cols, int8_t *qa,
+                                  float *sa, int64_t blocks_pad, bool t16, hipStream_t s) {
+  const int64_t tiles = t16 ? (m + 15) / 16 * (blocks_pad / 2) : (m + 31) / 32 * blocks_pad;
+  const dim3 grid((unsigned)((tiles + 3) / 4));
+  const int32_t nb = (int32_t)(cols / kBlock), np = (int32_t)blocks_pad;
+  if (t16)
+    hipLaunchKernelGGL((quantize_tiles_kernel<XB, AL, true>), grid, dim3(256), 0, s, x, m, ldx,
+                       nb, np, tiles, qa, sa);
+  else
+    hipLaunchKernelGGL((quantize_tiles_kernel<XB, AL, false>), grid, dim3(256), 0, s, x, m, ldx,
+                       nb, np, tiles, qa, sa);
+}
+
 hipError_t launch_quantize_tiled(const void *x, bool x_bf16, int64_t m,
                                  int64_t ldx, int64_t cols, int8_t *qa,
-                                 float *sa, int64_t blocks_pad, hipStream_t s) {
-  const int64_t blocks = cols / kBlock;
-  const int64_t tiles = (m + 31) / 32 * blocks_pad;
+                                 float *sa, int64_t blocks_pad, bool t16,
+                                 hipStream_t s) {
   const int64_t esz = x_bf16 ? 2 : 4;
-  const int aligned =
-      ((uintptr_t)x % (4 * esz) == 0) && (ldx % 4 == 0) ? 1 : 0;
-  const dim3 grid((unsigned)((tiles + 3) / 4));
-  const int32_t nb = (int32_t)blocks, np = (int32_t)blocks_pad;
-  if (x_bf16) {
-    if (aligned)
-      hipLaunchKernelGGL((quantize_tiles_kernel<true, true>), grid, dim3(256), 0, s, x, m, ldx, nb, np, tiles, qa, sa);
-    else
-      hipLaunchKernelGGL((quantize_tiles_kernel<true, false>), grid, dim3(256), 0, s, x, m, ldx, nb, np, tiles, qa, sa);
-  } else {
-    if (aligned)
-      hipLaunchKernelGGL((quantize_tiles_kernel<false, true>), grid, dim3(256), 0, s, x, m, ldx, nb, np, tiles, qa, sa);
-    else
-      hipLaunchKernelGGL((quantize_tiles_kernel<false, false>), grid, dim3(256), 0, s, x, m, ldx, nb, np, tiles, qa, sa);
-  }
+  const bool aligned = ((uintptr_t)x % (4 * esz) == 0) && (ldx % 4 == 0);
+  if (x_bf16)
+    aligned ? launch_quantize_tiles<true, true>(x, m, ldx, cols, qa, sa, blocks_pad, t16, s)
+            : launch_quantize_tiles<true, false>(x, m, ldx, cols, qa, sa, blocks_pad, t16, s);
+  else
+    aligned ? launch_quantize_tiles<false, true>(x, m, ldx, cols, qa, sa, blocks_pad, t16, s)
+            : launch_quantize_tiles<false, false>(x, m, ldx, cols, qa, sa, blocks_pad, t16, s);
   return hipGetLastError();
 }
 

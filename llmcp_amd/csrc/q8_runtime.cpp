@@ -1085,10 +1085,11 @@ static int gemm_operands_fit(const Tensor *w, int64_t m) {
   return LLMCP_Q8_OK;
 }
 
-// Q8_1 of the input rows into the workspace (the GEMM's tiled layout; the
-// context's scratch grows on first use for a larger M).
+// Q8_1 of the input rows into the workspace (the GEMM's tiled layout, 16-row
+// tiles for launch_gemm16; the context's scratch grows on first use for a
+// larger M).
 static int gemm_quantize(llmcp_q8_ctx *ctx, const Rows &in, const Tensor *w,
-                         Workspace &ws) {
+                         Workspace &ws, bool t16) {
   const int64_t m = in.rows;
   if (int rc = gemm_operands_fit(w, m)) return rc;
   const int64_t nblk = passes_for(w->cols) * kPassBlocks;
@@ -1097,8 +1098,54 @@ static int gemm_quantize(llmcp_q8_ctx *ctx, const Rows &in, const Tensor *w,
                    (uint64_t)(row_tiles * 32 * nblk * 4));
   if (rc) return rc;
   hipError_t e = launch_quantize_tiled(in.data, in.bf16, m, in.ld, w->cols,
-                                       ws.qa, ws.sa, nblk, ctx->stream);
+                                       ws.qa, ws.sa, nblk, t16, ctx->stream);
   if (e != hipSuccess) return hip_fail(e, "quantize launch");
+  return LLMCP_Q8_OK;
+}
+
+// Whether these rows take the 16 x 16-tile GEMM, for `count` weights in one
+// launch (outputs of one element type).  It sums in the serial block order,
+// so it serves both accumulation modes; only a forced split count (a test
+// hook) goes past it.
+static bool gemm16_for(llmcp_q8_ctx *ctx, int64_t m, int32_t count, const Tensor *const *w,
+                       const Rows *outs, bool dual = false) {
+  const bool split_k = ctx->accumulation == LLMCP_Q8_ACCUM_SPLIT_K;
+  if (split_k && ctx->test_splits > 0) return false;
+  int64_t rows[kMaxGroup];
+  for (int32_t i = 0; i < count; ++i) {
+    if (outs[i].bf16 != outs[0].bf16) return false;
+    rows[i] = w[i]->rows;
+  }
+  return gemm16_takes(m, rows, count, w[0]->cols, dual, split_k);
+}
+
+// The 16 x 16-tile GEMM of the quantized rows: `count` weights in one
+// launch, or (up non-null, count 1) the SwiGLU of w[0] and up.
+static int gemm16_launch(llmcp_q8_ctx *ctx, const Workspace &ws, int64_t m,
+                         const Tensor *const *w, const Tensor *up, const Rows *outs,
+                         const int32_t *acts, int32_t count, const Rows *residual = nullptr) {
+  Gemm16Launch g;
+  g.qa = ws.qa;
+  g.sa = ws.sa;
+  g.m = m;
+  g.cols = w[0]->cols;
+  g.fma = ctx->fma();
+  g.y_bf16 = outs[0].bf16;
+  if (residual) {
+    g.add = residual->data;
+    g.ldr = residual->ld;
+  }
+  g.count = count;
+  for (int32_t i = 0; i < count; ++i) {
+    g.w[i].w = w[i]->dev;
+    g.w[i].up = up ? up->dev : nullptr;
+    g.w[i].y = outs[i].data;
+    g.w[i].ldy = outs[i].ld;
+    g.w[i].rows = w[i]->rows;
+    g.w[i].activation = acts ? acts[i] : LLMCP_Q8_ACT_NONE;
+  }
+  hipError_t e = launch_gemm16(g, ctx->stream);
+  if (e != hipSuccess) return hip_fail(e, "gemm launch");
   return LLMCP_Q8_OK;
 }
 
@@ -1157,8 +1204,10 @@ static int gemm_common(llmcp_q8_ctx *ctx, const Rows &in, const Tensor *w,
                        const Rows &out, int activation,
                        const Workspace *fixed = nullptr, bool exact = false) {
   Workspace ws = fixed ? *fixed : ctx_workspace(ctx);
-  int rc = gemm_quantize(ctx, in, w, ws);
+  const bool t16 = gemm16_for(ctx, in.rows, 1, &w, &out);
+  int rc = gemm_quantize(ctx, in, w, ws, t16);
   if (rc) return rc;
+  if (t16) return gemm16_launch(ctx, ws, in.rows, &w, nullptr, &out, &activation, 1);
   return gemm_launch(ctx, ws, in.rows, w, out, activation, nullptr, 0, nullptr, exact);
 }
 
@@ -1222,7 +1271,9 @@ static int linear_add_impl(llmcp_q8_ctx *ctx, const Rows &in,
   if (m == 1)
     return gemv_common(ctx, in, w, nullptr, out, LLMCP_Q8_ACT_NONE, nullptr, &res);
   Workspace ws = ctx_workspace(ctx);
-  if ((rc = gemm_quantize(ctx, in, w, ws))) return rc;
+  const bool t16 = gemm16_for(ctx, m, 1, &w, &out);
+  if ((rc = gemm_quantize(ctx, in, w, ws, t16))) return rc;
+  if (t16) return gemm16_launch(ctx, ws, m, &w, nullptr, &out, nullptr, 1, &res);
   return gemm_launch(ctx, ws, m, w, out, LLMCP_Q8_ACT_NONE, nullptr, 0, &res);
 }
 
@@ -1263,7 +1314,9 @@ static int linear_group_run(llmcp_q8_ctx *ctx, const Rows &in, int32_t count,
     for (int32_t i = 0; i < count; ++i)
       if ((rc = gemm_operands_fit(w[i], m))) return rc;
     Workspace ws = ctx_workspace(ctx);
-    if (!prequantized && (rc = gemm_quantize(ctx, in, w[0], ws))) return rc;
+    const bool t16 = gemm16_for(ctx, m, count, w, outs);
+    if (!prequantized && (rc = gemm_quantize(ctx, in, w[0], ws, t16))) return rc;
+    if (t16) return gemm16_launch(ctx, ws, m, w, nullptr, outs, acts, count);
     for (int32_t i = 0; i < count; ++i)
       if ((rc = gemm_launch(ctx, ws, m, w[i], outs[i], act_of(i), nullptr, 0)))
         return rc;
@@ -1422,7 +1475,9 @@ static int rmsnorm_group_impl(llmcp_q8_ctx *ctx, const Rows &in, const NormWeigh
     return rc;
   hipError_t e = launch_rmsnorm(in.data, in.bf16, m, in.ld, in.cols, nw.data, nw.bf16, eps,
                                 zero_centered != 0, normed.data, normed.bf16, normed.ld,
-                                ws.qa, ws.sa, nblk, 2, ctx->stream, ctx->rmsnorm_skew);
+                                ws.qa, ws.sa, nblk,
+                                gemm16_for(ctx, m, count, w, outs) ? 1 : 2, ctx->stream,
+                                ctx->rmsnorm_skew);
   if (e != hipSuccess) return hip_fail(e, "rmsnorm launch");
   return linear_group_run(ctx, normed, count, w, outs, acts, true);
 }
@@ -1443,6 +1498,12 @@ static int swiglu_impl(llmcp_q8_ctx *ctx, const Rows &in,
   if (m == 0) return LLMCP_Q8_OK;
   if ((rc = set_device(ctx))) return rc;
   if (m == 1) return gemv_common(ctx, in, wg, wu, out, LLMCP_Q8_ACT_NONE, nullptr);
+  if (gemm16_for(ctx, m, 1, &wg, &out, true)) {
+    Workspace ws = ctx_workspace(ctx);
+    if ((rc = gemm_operands_fit(wu, m)) || (rc = gemm_quantize(ctx, in, wg, ws, true)))
+      return rc;
+    return gemm16_launch(ctx, ws, m, &wg, wu, &out, nullptr, 1);
+  }
   // Several rows: the input quantized once; the gate GEMM with SiLU, then the up
   // GEMM whose epilogue does the multiply (MulOpLowering,
   // LowerToLinalg.cpp:377-393) with the gate's output.  f32: the gate goes
@@ -1459,7 +1520,7 @@ static int swiglu_impl(llmcp_q8_ctx *ctx, const Rows &in,
     g.ld = wg->rows;
   }
   Workspace ws = ctx_workspace(ctx);
-  if ((rc = gemm_quantize(ctx, in, wg, ws))) return rc;
+  if ((rc = gemm_quantize(ctx, in, wg, ws, false))) return rc;
   if ((rc = gemm_launch(ctx, ws, m, wg, g, LLMCP_Q8_ACT_SILU, nullptr, 0)))
     return rc;
   return gemm_launch(ctx, ws, m, wu, out, LLMCP_Q8_ACT_NONE,
@@ -1548,6 +1609,12 @@ static int mlp_impl(llmcp_q8_ctx *ctx, const Rows &in,
       h.cols = h.ld = f;
       h.bf16 = out.bf16;
     }
+    if (gemm16_for(ctx, m, 1, &wg, &h, true)) {
+      Workspace ws = ctx_workspace(ctx);
+      if ((rc = gemm_quantize(ctx, in, wg, ws, true))) return rc;
+      if ((rc = gemm16_launch(ctx, ws, m, &wg, wu, &h, nullptr, 1))) return rc;
+      return gemm_common(ctx, h, wd, out, LLMCP_Q8_ACT_NONE);
+    }
     Rows g = h;  // the gate's output: h itself (f32) or f32 scratch (bf16)
     if (h.bf16) {
       if ((rc = grow(ctx, ctx->up, ctx->up_bytes, (uint64_t)(m * f) * 4,
@@ -1558,7 +1625,7 @@ static int mlp_impl(llmcp_q8_ctx *ctx, const Rows &in,
       g.ld = f;
     }
     Workspace ws = ctx_workspace(ctx);
-    if ((rc = gemm_quantize(ctx, in, wg, ws))) return rc;
+    if ((rc = gemm_quantize(ctx, in, wg, ws, false))) return rc;
     if ((rc = gemm_launch(ctx, ws, m, wg, g, LLMCP_Q8_ACT_SILU, nullptr, 0)))
       return rc;
     if ((rc = gemm_launch(ctx, ws, m, wu, h, LLMCP_Q8_ACT_NONE,
