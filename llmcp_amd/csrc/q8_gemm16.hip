@@ -60,9 +60,9 @@ struct Gemm16Args {
 // units), per column tile the values and then the scale blocks.
 template <int SEG, int RT, int CN, bool DUAL>
 struct Gemm16Shape {
-  static constexpr int NT = DUAL ? 2 : 1;          // tiles per compute wave
-  static constexpr int CB = CN * NT;               // column tiles of B
-  static constexpr int W = RT * CN;                // compute waves
+  static constexpr int NM = DUAL ? 2 : 1;          // matrices
+  static constexpr int CB = CN * NM;               // column tiles of B
+  static constexpr int W = RT * CB;                // compute waves
   static constexpr int P = W > 4 || CB >= 4 ? 2 : 1;  // producers of A, and of B
   static constexpr int SB = SEG == 6 ? 24 : 16;    // blocks per weight stage
   static constexpr int SUB = SB / 8;               // A stages per weight stage
@@ -79,8 +79,12 @@ struct Gemm16Shape {
   static constexpr int BSZ = CB * TILE;
   // Ring depths: as deep as the LDS allows (weights come from HBM, and a
   // stage has the time of NB - 1 others to land), within unrolled loops of
-  // eight A stages (S = 6: nine).
-  static constexpr bool fits(int na, int nb) { return na * ASZ + nb * BSZ <= 160 * 1024; }
+  // eight A stages (S = 6: nine).  The SwiGLU pair of one row tile leaves
+  // room for three workgroups per CU instead: at N = 9216 that puts all 576
+  // in flight at once (19.3 us against 25.9 with four pairs of tiles in 144
+  // deep workgroups, M = 16, K = 2560; 17.7 with the non-temporal loads).
+  static constexpr int BUDGET = (DUAL && RT == 1 ? 53 : 160) * 1024;
+  static constexpr bool fits(int na, int nb) { return na * ASZ + nb * BSZ <= BUDGET; }
   static constexpr int NA = SEG != 6 && (fits(4, 4) || (!fits(3, 3) && fits(4, 2))) ? 4 : 3;
   static constexpr int NB = SEG != 6 && fits(4, 4) ? 4 : fits(3, 3) ? 3 : 2;
   static constexpr int BOFF = NA * ASZ;
@@ -129,21 +133,23 @@ __device__ __forceinline__ const uint8_t *uniform_base(const void *p) {
   return (const uint8_t *)(((uint64_t)hi << 32) | lo);
 }
 
-// Compute waves run a sequence of steps, one per quad of four blocks (and
-// matrix, if DUAL: the SwiGLU pair, the same 16 columns of both).  Entering
-// step k a wave holds step k's dots and scale tiles and step k+1's
+// Compute waves run a sequence of steps, one per quad of four blocks, two per
+// A stage.  Entering step k a wave holds step k's dots and scale tiles and step k+1's
 // operands; it issues step k+1's MFMAs and the LDS reads of step k+2's
 // operands, and then runs step k's 32-operation epilogue, which covers
-// both.  Two steps before the end of A stage t every operand of the stage
-// has been taken by an MFMA, so there the workgroup's barrier hands stage
-// t + 1 to the compute waves and stage t's buffer back to the producers.
+// both.  In the first step of A stage t every operand of the stage has been
+// taken by an MFMA, so there the workgroup's barrier hands stage t + 1 to the
+// compute waves and stage t's buffer back to the producers.
+// DUAL, the SwiGLU pair: a wave for the tile of the gate matrix and one for
+// the same columns of the up matrix, which hands its sums over through LDS
+// at the end.
 template <int SEG, bool FMA, int RT, int CN, bool DUAL>
 __global__ __launch_bounds__((Gemm16Shape<SEG, RT, CN, DUAL>::BOUND))
 void gemm16_kernel(const Gemm16Args p) {
 #ifdef __HIP_DEVICE_COMPILE__  // the host pass needs the stub only (and drops
                                // it where it meets the operand pins below)
   typedef Gemm16Shape<SEG, RT, CN, DUAL> Sh;
-  constexpr int NT = Sh::NT, NA = Sh::NA, NB = Sh::NB, SUB = Sh::SUB;
+  constexpr int NM = Sh::NM, NA = Sh::NA, NB = Sh::NB, SUB = Sh::SUB;
   __shared__ __align__(1024) uint8_t smem[Sh::LDS];
 
   // all row groups of a column group on one XCD (ids equal modulo 8)
@@ -261,10 +267,15 @@ void gemm16_kernel(const Gemm16Args p) {
           const auto r = rsrc_of(base[u], s < bstages);
           const auto to = (lds_void *)(smem + Sh::BOFF + buf * Sh::BSZ + dst[u]);
           const uint32_t off = unit * kPassBytes + uoff[u] + quarter * uslot[u];
+          // up to 16 rows one workgroup alone reads these weights: non-temporal
+          // (M = 16, N = 9216, K = 2560 13.9 -> 12.9 us from HBM; at 32 rows
+          // 4 % less from HBM, 10 % more for weights that fit the 256 MB
+          // cache behind it)
+          constexpr int kNt = RT == 1 ? 2 : 0;
           if constexpr (u < Sh::DQ || SEG == 1)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, to, 16, voff[u], off, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, to, 16, voff[u], off, 0, kNt);
           else
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, to, 4, voff[u], off, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, to, 4, voff[u], off, 0, kNt);
         });
       };
 #pragma unroll
@@ -280,16 +291,20 @@ void gemm16_kernel(const Gemm16Args p) {
         buf = buf + 1 == NB ? 0 : buf + 1;
       }
     }
-    // no DMA may land in LDS after the workgroup has released it
+    // no DMA may land in LDS after the workgroup has released it (or, with
+    // DUAL, after the compute waves have taken the rings for their sums)
     wait_vmcnt16<0>();
+    if constexpr (DUAL) barrier16();
     return;
   }
 
   // ---- compute waves
-  const int wr = wave % RT, wc = wave / RT;
+  const int wr = wave % RT, wt = wave / RT;  // its row tile and tile of B
+  const int wc = wt / NM;
   const int rt16 = mg * RT + wr;  // this wave's 16-row tile
   if ((int64_t)rt16 * 16 >= p.m_rows) {
     for (int t = 0; t <= stages; ++t) barrier16();
+    if constexpr (DUAL) barrier16();
     return;
   }
   const int li = lane & 15, lq = lane >> 4;
@@ -306,7 +321,7 @@ void gemm16_kernel(const Gemm16Args p) {
                  (((2 * j + (lq >> 1)) ^ li) << 4);
     else
       baddr[j] = (lq & 1) * 1024 + (lq >> 1) * 2048 + li * 64 + ((j ^ (li >> 2)) << 4);
-    baddr[j] += Sh::BOFF + wc * NT * Sh::TILE;
+    baddr[j] += Sh::BOFF + wt * Sh::TILE;
   }
   // weight scales: lane (row li, block 4q + lq of the weight stage)
   constexpr int QB = Sh::SB / 4;  // quads per weight stage
@@ -315,7 +330,7 @@ void gemm16_kernel(const Gemm16Args p) {
   for (int q = 0; q < (SEG == 6 ? QB : 1); ++q) {
     const int e = 4 * q + lq;
     const int i = SEG == 1 ? 0 : e % SEG, sl = SEG == 1 ? e : e / SEG;
-    daddr[q] = Sh::BOFF + wc * NT * Sh::TILE + Sh::QOPS * 1024 +
+    daddr[q] = Sh::BOFF + wt * Sh::TILE + Sh::QOPS * 1024 +
                (SEG == 1 ? (li >> 2) * 128 + 2 * (16 * (li & 3) + sl) : i * 128 + li * 8 + 2 * sl);
   }
 
@@ -323,18 +338,16 @@ void gemm16_kernel(const Gemm16Args p) {
   v4i fa[2], fb[2];
   float fs;
   uint16_t fd;
-  // Operands of the step of the A stage at place T of the unrolled rings, its
-  // quad Q (0, 1) and matrix M.
-  auto read_ops = [&](auto T, auto Q, auto M) __attribute__((always_inline)) {
-    constexpr int T_ = decltype(T)::value, q = decltype(Q)::value, m = decltype(M)::value;
+  // Operands of the step of the A stage at place T of the unrolled rings and
+  // its quad Q (0, 1).
+  auto read_ops = [&](auto T, auto Q) __attribute__((always_inline)) {
+    constexpr int T_ = decltype(T)::value, q = decltype(Q)::value;
     constexpr int a0 = T_ % NA * Sh::ASZ;
-    constexpr int b0 = T_ / SUB % NB * Sh::BSZ + m * Sh::TILE;
+    constexpr int b0 = T_ / SUB % NB * Sh::BSZ;
     constexpr int qb = T_ % SUB * 2 + q;  // quad of the weight stage
-    if constexpr (m == 0) {
 #pragma unroll
-      for (int j = 0; j < 2; ++j) fa[j] = *(const v4i *)(smem + aaddr + (a0 + (2 * q + j) * 1024));
-      fs = *(const float *)(smem + saddr + (a0 + q * 256));
-    }
+    for (int j = 0; j < 2; ++j) fa[j] = *(const v4i *)(smem + aaddr + (a0 + (2 * q + j) * 1024));
+    fs = *(const float *)(smem + saddr + (a0 + q * 256));
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int e = 4 * qb + 2 * j;  // the pair's even block
@@ -347,11 +360,7 @@ void gemm16_kernel(const Gemm16Args p) {
 
   v4i cc[4], cn[4];
   v16f fc, fn;
-  float acc[NT][4];
-#pragma unroll
-  for (int t = 0; t < NT; ++t)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) acc[t][v] = 0.0f;
+  float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
   // Lanes 0-31 of fb hold the even block of the pair (both halves of its
   // values), lanes 32-63 the odd one: swapping the upper lanes of the first
   // eight bytes with the lower lanes of the last eight gives each block an
@@ -375,19 +384,16 @@ void gemm16_kernel(const Gemm16Args p) {
     return __builtin_amdgcn_mfma_f32_16x16x1f32(fs, half_bits_to_float(fd), z, 0, 0, 0);
   };
 
-  constexpr int KN = 2 * NT;  // steps per A stage
   auto stage_steps = [&](auto T) __attribute__((always_inline)) {
-    static_for<KN>([&](auto K) __attribute__((always_inline)) {
-      constexpr int k = decltype(K)::value, T_ = decltype(T)::value;
-      constexpr int k2 = (k + 2) % KN, d2 = (k + 2) / KN;
+    static_for<2>([&](auto K) __attribute__((always_inline)) {
+      constexpr int T_ = decltype(T)::value;
       dots(cn);
       fn = scales();
 #pragma unroll
       for (int j = 0; j < 4; ++j) asm volatile("" ::"v"(cn[j]));
       asm volatile("" ::"v"(fn));
-      if constexpr (k == KN - 2) barrier16();
-      read_ops(std::integral_constant<int, (T_ + d2) % Sh::PERIOD>{},
-               std::integral_constant<int, k2 / NT>{}, std::integral_constant<int, k2 % NT>{});
+      if constexpr (decltype(K)::value == 0) barrier16();
+      read_ops(std::integral_constant<int, (T_ + 1) % Sh::PERIOD>{}, K);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int j = 0; j < 4; ++j)
@@ -395,16 +401,15 @@ void gemm16_kernel(const Gemm16Args p) {
         for (int v = 0; v < 4; ++v) {
           const float dotf = (float)cc[j][v];
           const float f = fc[4 * j + v];
-          float &a = acc[k % NT][v];
           if (FMA) {
-            a = __builtin_fmaf(dotf, f, a);
+            acc[v] = __builtin_fmaf(dotf, f, acc[v]);
           } else {
             const float contrib = dotf * f;
-            a = a + contrib;
+            acc[v] = acc[v] + contrib;
           }
         }
 #pragma unroll
-      for (int v = 0; v < 4; ++v) asm volatile("" : "+v"(acc[k % NT][v]));
+      for (int v = 0; v < 4; ++v) asm volatile("" : "+v"(acc[v]));
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int j = 0; j < 4; ++j) cc[j] = cn[j];
@@ -415,10 +420,11 @@ void gemm16_kernel(const Gemm16Args p) {
   barrier16();
   {
     using I0 = std::integral_constant<int, 0>;
-    read_ops(I0{}, I0{}, I0{});
+    using I1 = std::integral_constant<int, 1>;
+    read_ops(I0{}, I0{});
     dots(cc);
     fc = scales();
-    read_ops(I0{}, std::integral_constant<int, 1 / NT>{}, std::integral_constant<int, 1 % NT>{});
+    read_ops(I0{}, I1{});
   }
   for (int t0 = 0; t0 < stages; t0 += Sh::PERIOD)
     static_for<Sh::PERIOD>([&](auto T) __attribute__((always_inline)) {
@@ -426,20 +432,34 @@ void gemm16_kernel(const Gemm16Args p) {
       if (t < stages) stage_steps(T);
     });
 
+  typedef float v4f __attribute__((ext_vector_type(4)));
+  float up[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  if constexpr (DUAL) {
+    // every DMA has landed and every operand has been read: the up waves'
+    // sums take the rings' place
+    barrier16();
+    v4f *const box = (v4f *)(smem + (wc * RT + wr) * 1024 + lane * 16);
+    if (wt & 1) {
+      *box = v4f{acc[0], acc[1], acc[2], acc[3]};
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    }
+    barrier16();
+    if (wt & 1) return;
+    const v4f u = *box;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) up[v] = u[v];
+  }
+
   const int n = nc0 + 16 * wc + li;
   const int64_t m0 = (int64_t)rt16 * 16 + 4 * lq;
   float o[4];
-  if constexpr (DUAL) {
-    activate_array(acc[0], ACT_SILU);
+  activate_array(acc, DUAL ? ACT_SILU : gw.act);
 #pragma unroll
-    for (int v = 0; v < 4; ++v)
-      o[v] = p.y_bf16 ? bf16_to_float(float_to_bf16(acc[0][v])) *
-                            bf16_to_float(float_to_bf16(acc[NT - 1][v]))
-                      : acc[0][v] * acc[NT - 1][v];
-  } else {
-    activate_array(acc[0], gw.act);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) o[v] = acc[0][v];
+  for (int v = 0; v < 4; ++v) {
+    o[v] = acc[v];
+    if constexpr (DUAL)
+      o[v] = p.y_bf16 ? bf16_to_float(float_to_bf16(o[v])) * bf16_to_float(float_to_bf16(up[v]))
+                      : o[v] * up[v];
   }
 #pragma unroll
   for (int v = 0; v < 4; ++v) {
@@ -478,10 +498,10 @@ hipError_t launch16(Gemm16Args &a, const Gemm16Launch &l, int32_t row_tiles16, h
 // fewest columns that put every workgroup on a CU of its own.  `per_block`
 // is a round's time per block of K, in us, fitted with 5 us of launch, fill
 // and input quantization to op times at N = 1000 .. 9216 (f32, aarch64):
-// (1, 1) 10.1 us at K = 2560, 18.9 at 9216; (1, 4) 14.0 at N = 9216, K =
+// (1, 1) 9.6 us at K = 2560, 18.6 at 9216; (1, 4) 12.9 at N = 9216, K =
 // 2560; (4, 1) 10.9 / 14.0 / 23.9 at K = 2560 / 4096 / 9216; (4, 2) 13.7 /
-// - / 33; (4, 3) 16.7 / 23.2 / 43.8; SwiGLU (1, 4) 24.9, (2, 3) 24.3, (4, 1)
-// 15.8 at K = 2560.
+// - / 33; (4, 3) 16.7 / 23.2 / 43.8; SwiGLU (1, 1) 12.4 at N = 2560, 17.5 at
+// 9216, (2, 3) 23.2, (4, 1) 15.2 .. 16.7 at K = 2560.
 struct Shape16 {
   int rt, cn;
   double per_block;
@@ -489,11 +509,8 @@ struct Shape16 {
 Shape16 shape16(int64_t rts, int64_t tiles, int seg, bool dual) {
   const int64_t cus = cu_count();
   if (dual) {
-    // 4 (3) column pairs do not fit the LDS with S = 6
-    if (rts == 1) {
-      if (tiles <= cus) return {1, 1, 0.10};
-      return tiles <= 2 * cus || seg == 6 ? Shape16{1, 2, 0.14} : Shape16{1, 4, 0.25};
-    }
+    if (rts == 1) return {1, 1, 0.06};
+    // three column pairs do not fit the LDS with S = 6
     if (rts == 2) return tiles <= cus || seg == 6 ? Shape16{2, 1, 0.11} : Shape16{2, 3, 0.24};
     return {4, 1, 0.14};
   }
@@ -503,11 +520,11 @@ Shape16 shape16(int64_t rts, int64_t tiles, int seg, bool dual) {
   }
   if (rts == 2) {
     if (tiles <= cus) return {2, 1, 0.055};
-    return tiles <= 2 * cus ? Shape16{2, 2, 0.08} : Shape16{2, 4, 0.135};
+    return tiles <= 2 * cus ? Shape16{2, 2, 0.08} : Shape16{2, 4, 0.15};
   }
   const int64_t wgs = (rts + 3) / 4 * tiles;
   if (wgs <= cus) return {4, 1, 0.065};
-  return wgs <= 2 * cus ? Shape16{4, 2, 0.10} : Shape16{4, 3, 0.15};
+  return wgs <= 2 * cus ? Shape16{4, 2, 0.10} : Shape16{4, 3, 0.14};
 }
 
 // Rounds of workgroups, at most one per CU.
@@ -524,14 +541,11 @@ hipError_t launch16_f(Gemm16Args &a, const Gemm16Launch &l, int32_t rts, const S
   if (dual) {
     switch (code) {
       case 11: return launch16<SEG, FMA, 1, 1, true>(a, l, rts, s);
-      case 12: return launch16<SEG, FMA, 1, 2, true>(a, l, rts, s);
       case 21: return launch16<SEG, FMA, 2, 1, true>(a, l, rts, s);
       case 41: return launch16<SEG, FMA, 4, 1, true>(a, l, rts, s);
     }
-    if constexpr (SEG != 6) {
-      if (code == 14) return launch16<SEG, FMA, 1, 4, true>(a, l, rts, s);
+    if constexpr (SEG != 6)
       if (code == 23) return launch16<SEG, FMA, 2, 3, true>(a, l, rts, s);
-    }
     return hipErrorInvalidValue;
   }
   switch (code) {
@@ -551,15 +565,17 @@ hipError_t launch16_f(Gemm16Args &a, const Gemm16Launch &l, int32_t rts, const S
 }  // namespace
 
 // The cheaper of the two GEMMs by the fitted op times.  launch_gemm, exact:
-// up to 64 rows 1 + 0.18 us per block for each 256 of its 64 x 64 workgroups
-// (14.2 .. 15.9 us at K = 2560, 26 at 4096, 54 at 9216), above 0.33 us per
+// up to 64 rows 1 + 0.18 us per block for one 64 x 64 workgroup per CU (14.2
+// .. 15.9 us at K = 2560, 26 at 4096, 54 at 9216) and 1 + 0.28 for each two
+// (178 us at N = 248320, K = 2560, M = 32), above 0.33 us per
 // block and round of 128 x 96 ones (25 .. 30 us at K = 2560, 45 at 4096, 105
 // at 9216), for each weight apart.  Op times launch_gemm -> launch_gemm16:
 // N = 2560, K = 9216 M = 2 / 64 / 256 / 512 53.8 / 56.2 / 105.6 / 105.0 ->
 // 18.9 / 23.9 / 43.8 / 81.1; N = 2560, K = 2560 M = 64 / 256 / 320 14.2 /
 // 26.0 / 26.2 -> 10.9 / 16.7 / 27.1 (not taken); N = 9216, K = 2560 M = 16 /
-// 32 / 64 15.4 / 15.7 / 15.8 -> 14.0 / 15.7 / 18.2 (the last two not taken);
-// its SwiGLU M = 16 / 32 29.2 / 30.0 -> 24.9 / 24.3.
+// 32 / 64 15.4 / 15.7 / 15.8 -> 12.9 / 15.8 / 18.2 (the last two not taken);
+// its SwiGLU M = 16 / 32 29.6 / 30.3 -> 17.5 / 23.3; N = 2560, K = 9216 / 4096
+// M = 333 104.9 / 45.4 -> 73.6 / 38.1.
 // Where K may be split (split_k) a second round loses to the splits (N =
 // 2560, K = 9216, M = 512: 73 us), one round does not (M = 256: 50).
 bool gemm16_takes(int64_t m, const int64_t *rows, int count, int64_t cols, bool dual,
@@ -572,13 +588,15 @@ bool gemm16_takes(int64_t m, const int64_t *rows, int count, int64_t cols, bool 
   for (int i = 0; i < count; ++i) {
     tiles += (rows[i] + 15) / 16;
     const int64_t wgs = m <= 64 ? (rows[i] + 63) / 64 : (m + 127) / 128 * ((rows[i] + 95) / 96);
-    const double rounds = (double)((wgs + cus - 1) / cus);
-    old_us += rounds * (m <= 64 ? 1.0 + 0.18 * blocks : 0.33 * blocks) * (dual ? 2 : 1);
+    const double us = m > 64     ? (double)((wgs + cus - 1) / cus) * 0.33 * blocks
+                      : wgs <= cus ? 1.0 + 0.18 * blocks
+                                   : (double)((wgs + 2 * cus - 1) / (2 * cus)) * (1.0 + 0.28 * blocks);
+    old_us += us * (dual ? 2 : 1);
   }
   const Shape16 sh = shape16(rts, tiles, seg_for(units), dual);
   const int64_t rounds = rounds16(sh, rts, tiles);
   if (split_k && rounds > 1) return false;
-  return (double)rounds * (5.0 + sh.per_block * blocks) < old_us;
+  return 5.0 + (double)rounds * sh.per_block * blocks < old_us;
 }
 
 hipError_t launch_gemm16(const Gemm16Launch &l, hipStream_t s) {
