@@ -944,6 +944,123 @@ __global__ __launch_bounds__(512) void gated_rmsnorm_kernel(
   }
 }
 
+// The same for many groups of up to kGatedManyG values: sixteen per
+// workgroup, four waves that load x, gate and weight, write the squares to
+// LDS and form p, and a fifth whose lanes fold a group each (rows of g + 4
+// floats, so that sixteen lanes' 16 B reads fall in different banks).  A fold
+// by a whole wave takes a wave slot for 128 dependent additions per group:
+// bound by rounds of workgroups, 10656 groups of 128 (333 rows of 4096, bf16)
+// took 11.2 us so, 6.8 here (26 MB: 3.9 TB/s).
+constexpr int kGatedManyG = 256;
+constexpr int kGatedMany = 16;                     // groups per workgroup
+constexpr int kGatedManySlots = kGatedManyG * kGatedMany / 4 / 256;  // float4s per lane
+
+template <bool XB>
+__global__ __launch_bounds__(320) void gated_rmsnorm_many_kernel(
+    const void *__restrict__ x, const void *__restrict__ gate, const float *__restrict__ w,
+    int64_t groups, int32_t g, float eps, int gate_activated, void *__restrict__ y,
+    int aligned) {
+  __shared__ __align__(16) float sq[kGatedMany * (kGatedManyG + 4)];
+  __shared__ float rstd[kGatedMany];
+  const int t = threadIdx.x, g4 = g / 4;
+  const int64_t grp0 = (int64_t)blockIdx.x * kGatedMany;
+  const int n4 = (int)min((int64_t)kGatedMany, groups - grp0) * g4;  // float4s here
+  asm volatile("" ::"s"(y), "s"(eps), "s"(gate_activated));
+  uint4 rx[kGatedManySlots], rg[kGatedManySlots];
+  float4 pv[kGatedManySlots];
+  auto load = [&](auto al) __attribute__((always_inline)) {
+    constexpr bool AL = decltype(al)::value;
+#pragma unroll
+    for (int k = 0; k < kGatedManySlots; ++k) {
+      const int f = t + 256 * k;
+      if (f < n4) {
+        rx[k] = load_raw4<XB, AL>(x, grp0 * g + 4 * f);
+        rg[k] = load_raw4<XB, AL>(gate, grp0 * g + 4 * f);
+        pv[k] = *(const float4 *)(w + 4 * (f % g4));
+      }
+    }
+  };
+  if (t < 256) {
+    if (aligned & 1)
+      load(std::true_type{});
+    else
+      load(std::false_type{});
+#pragma unroll
+    for (int k = 0; k < kGatedManySlots; ++k) {
+      const int f = t + 256 * k;
+      if (f < n4) {
+        const float4 v = act4_of_raw<XB>(rx[k]);
+        *(float4 *)&sq[f / g4 * (g + 4) + 4 * (f % g4)] =
+            make_float4(v.x * v.x, v.y * v.y, v.z * v.z, v.w * v.w);
+      }
+    }
+  }
+  __syncthreads();
+  if (t >= 256) {
+    const int j = t & (kGatedMany - 1);
+    const float sum = fold_serial(sq + j * (g + 4), g, 0.0f);
+    const float mean = sum / (float)g;
+    const float var = mean + eps;
+    if (t < 256 + kGatedMany) rstd[j] = 1.0f / sqrtf(var);
+  } else {
+#pragma unroll
+    for (int k = 0; k < kGatedManySlots; ++k) {
+      if (t + 256 * k < n4) {
+        const float4 xv = act4_of_raw<XB>(rx[k]);
+        float4 gv = act4_of_raw<XB>(rg[k]);
+        if (!gate_activated) {
+          gv.x = silu_f32(gv.x);
+          gv.y = silu_f32(gv.y);
+          gv.z = silu_f32(gv.z);
+          gv.w = silu_f32(gv.w);
+        }
+        pv[k].x = (xv.x * gv.x) * pv[k].x;
+        pv[k].y = (xv.y * gv.y) * pv[k].y;
+        pv[k].z = (xv.z * gv.z) * pv[k].z;
+        pv[k].w = (xv.w * gv.w) * pv[k].w;
+      }
+    }
+  }
+  __syncthreads();
+  if (t >= 256) return;
+#pragma unroll
+  for (int k = 0; k < kGatedManySlots; ++k) {
+    const int f = t + 256 * k;
+    if (f < n4) {
+      const float rs = rstd[f / g4];
+      float4 v;
+      v.x = pv[k].x * rs;
+      v.y = pv[k].y * rs;
+      v.z = pv[k].z * rs;
+      v.w = pv[k].w * rs;
+      if constexpr (XB) {
+        const uint16_t h0 = float_to_bf16(v.x), h1 = float_to_bf16(v.y),
+                       h2 = float_to_bf16(v.z), h3 = float_to_bf16(v.w);
+        uint16_t *yp = (uint16_t *)y + grp0 * g + 4 * f;
+        if (aligned & 2) {
+          *(uint2 *)yp = make_uint2((uint32_t)h0 | ((uint32_t)h1 << 16),
+                                    (uint32_t)h2 | ((uint32_t)h3 << 16));
+        } else {
+          yp[0] = h0;
+          yp[1] = h1;
+          yp[2] = h2;
+          yp[3] = h3;
+        }
+      } else {
+        float *yp = (float *)y + grp0 * g + 4 * f;
+        if (aligned & 2) {
+          *(float4 *)yp = v;
+        } else {
+          yp[0] = v.x;
+          yp[1] = v.y;
+          yp[2] = v.z;
+          yp[3] = v.w;
+        }
+      }
+    }
+  }
+}
+
 // First-maximum argmax of one f32 row already in HBM (the last row of a
 // prefill lm_head's logits): the same keys as the GEMV's fused argmax,
 // folded into the same slots, so argmax_reduce_kernel finishes it.  A grid
@@ -1315,8 +1432,23 @@ hipError_t launch_gated_rmsnorm(const void *x, const void *gate, bool bf16,
   const dim3 grid((unsigned)((groups + kNormRows - 1) / kNormRows));
   const int32_t gg = (int32_t)g;
   const int ga = gate_activated ? 1 : 0;
+  const int yal = (uintptr_t)y % (4 * esz) == 0 ? 2 : 0;
+  // Many groups per launch pay off once the groups of four outnumber the
+  // resident workgroups (bf16, us, four / sixteen per workgroup: groups of 32
+  // 2.9 / 3.0 at 512, 3.5 / 3.0 at 2048, 10.3 / 3.4 at 10656; of 128 3.5 / 4.4
+  // at 2048, 5.3 / 4.5 at 4096, 31.0 / 16.6 at 32768; of 256 6.2 / 7.3 at 4096,
+  // 14.8 / 12.0 at 10656).
+  if (g <= kGatedManyG && groups >= std::max<int64_t>(2048, 32 * g)) {
+    const dim3 many((unsigned)((groups + kGatedMany - 1) / kGatedMany));
+    if (bf16)
+      hipLaunchKernelGGL(gated_rmsnorm_many_kernel<true>, many, dim3(320), 0, s, x, gate, w,
+                         groups, gg, eps, ga, y, aligned | yal);
+    else
+      hipLaunchKernelGGL(gated_rmsnorm_many_kernel<false>, many, dim3(320), 0, s, x, gate, w,
+                         groups, gg, eps, ga, y, aligned | yal);
+    return hipGetLastError();
+  }
   if (g <= kGatedMaxG) {
-    const int yal = (uintptr_t)y % (4 * esz) == 0 ? 2 : 0;
     const size_t lds = (size_t)4 * g * sizeof(float);
     if (bf16)
       hipLaunchKernelGGL(gated_rmsnorm_kernel<true>, grid, dim3(512), lds, s, x, gate, w,
