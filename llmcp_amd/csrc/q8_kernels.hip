@@ -256,14 +256,18 @@ __global__ void quantize_kernel(const void *__restrict__ x, int x_bf16,
 // one block: lane l takes values 4(l%8) .. +3 of its row, so each step reads
 // eight 128 B runs.  quantize_block8 does the arithmetic, so the bits match
 // the row kernel.  Rows past m and blocks past `blocks` are written as zeros.
-template <bool XB, bool AL, bool T16>
+// STEPS: the steps that one wave takes, all four, or one where the tiles are
+// few and the launch is bound by a wave's latency.
+template <bool XB, bool AL, bool T16, int STEPS>
 __global__ __launch_bounds__(256) void quantize_tiles_kernel(
     const void *__restrict__ x, int64_t m, int64_t ldx, int32_t blocks,
     int32_t blocks_pad, int64_t tiles, int8_t *__restrict__ qa,
     float *__restrict__ sa) {
   const int lane = threadIdx.x & 63;
-  const int64_t tile = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int64_t unit = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int64_t tile = unit / (4 / STEPS);
   if (tile >= tiles) return;  // uniform per wave
+  const int c0 = (int)(unit - tile * (4 / STEPS)) * STEPS;  // the wave's first step
   const int32_t per_row = T16 ? blocks_pad / 2 : blocks_pad;
   const int32_t rt = (int32_t)(tile / per_row);
   const int32_t b0 = (int32_t)(tile - (int64_t)rt * per_row) * (T16 ? 2 : 1);
@@ -271,26 +275,29 @@ __global__ __launch_bounds__(256) void quantize_tiles_kernel(
   // step c's row within the tile and its block
   auto row_of = [&](int c) { return T16 ? 8 * (c >> 1) + rr : 8 * c + rr; };
   auto block_of = [&](int c) { return T16 ? b0 + (c & 1) : b0; };
-  // The four loads go out unconditionally (rows past m and padded blocks
+  // The loads go out unconditionally (rows past m and padded blocks
   // read a clamped address) and are zeroed only once all are in flight.
-  float4 v[4];
+  float4 v[STEPS];
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
+  for (int u = 0; u < STEPS; ++u) {
+    const int c = c0 + u;
     const int64_t row = (int64_t)rt * (T16 ? 16 : 32) + row_of(c);
     const int64_t rc = row < m ? row : m - 1;
     const int32_t bc = block_of(c) < blocks ? block_of(c) : blocks - 1;
-    v[c] = load_act4_t<XB, AL>(x, rc * ldx + (int64_t)bc * kBlock + 4 * p);
+    v[u] = load_act4_t<XB, AL>(x, rc * ldx + (int64_t)bc * kBlock + 4 * p);
   }
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
+  for (int u = 0; u < STEPS; ++u) {
+    const int c = c0 + u;
     const int64_t row = (int64_t)rt * (T16 ? 16 : 32) + row_of(c);
-    if (!(row < m && block_of(c) < blocks)) v[c] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (!(row < m && block_of(c) < blocks)) v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
   }
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
+  for (int u = 0; u < STEPS; ++u) {
+    const int c = c0 + u;
     int32_t q;
     float s;
-    quantize_block8(v[c], true, &q, &s);
+    quantize_block8(v[u], true, &q, &s);
     const int r = row_of(c);
     const int32_t off = T16 ? tile16_offset(r, c & 1, 4 * p) : r * kBlock + 4 * p;
     *(int32_t *)(qa + tile * 1024 + off) = q;
@@ -1286,18 +1293,33 @@ hipError_t launch_quantize(const void *x, bool x_bf16, int64_t m, int64_t ldx,
   return hipGetLastError();
 }
 
-template <bool XB, bool AL>
+template <bool XB, bool AL, bool T16>
 static void launch_quantize_tiles(const void *x, int64_t m, int64_t ldx, int64_t cols, int8_t *qa,
-                                  float *sa, int64_t blocks_pad, bool t16, hipStream_t s) {
-  const int64_t tiles = t16 ? (m + 15) / 16 * (blocks_pad / 2) : (m + 31) / 32 * blocks_pad;
-  const dim3 grid((unsigned)((tiles + 3) / 4));
+                                  float *sa, int64_t blocks_pad, hipStream_t s) {
+  const int64_t tiles = T16 ? (m + 15) / 16 * (blocks_pad / 2) : (m + 31) / 32 * blocks_pad;
   const int32_t nb = (int32_t)(cols / kBlock), np = (int32_t)blocks_pad;
-  if (t16)
-    hipLaunchKernelGGL((quantize_tiles_kernel<XB, AL, true>), grid, dim3(256), 0, s, x, m, ldx,
-                       nb, np, tiles, qa, sa);
+  // Up to a tile per SIMD, four waves each (op times, four steps -> one a wave:
+  // N = 2560 K = 2560 M = 2 / 64 / 256 8.6 / 10.9 / 16.4 -> 8.1 / 10.3 / 15.9 us);
+  // with more, the waves are enough either way (M = 1024 32.9 / 32.4 at K =
+  // 2560, 116 / 120 in bf16 at K = 9216).
+  if (tiles <= 4 * cu_count())
+    hipLaunchKernelGGL((quantize_tiles_kernel<XB, AL, T16, 1>), dim3((unsigned)tiles), dim3(256),
+                       0, s, x, m, ldx, nb, np, tiles, qa, sa);
   else
-    hipLaunchKernelGGL((quantize_tiles_kernel<XB, AL, false>), grid, dim3(256), 0, s, x, m, ldx,
-                       nb, np, tiles, qa, sa);
+    hipLaunchKernelGGL((quantize_tiles_kernel<XB, AL, T16, 4>), dim3((unsigned)((tiles + 3) / 4)),
+                       dim3(256), 0, s, x, m, ldx, nb, np, tiles, qa, sa);
+}
+
+template <bool T16>
+static void launch_quantize_layout(const void *x, bool x_bf16, bool aligned, int64_t m, int64_t ldx,
+                                   int64_t cols, int8_t *qa, float *sa, int64_t blocks_pad,
+                                   hipStream_t s) {
+  if (x_bf16)
+    aligned ? launch_quantize_tiles<true, true, T16>(x, m, ldx, cols, qa, sa, blocks_pad, s)
+            : launch_quantize_tiles<true, false, T16>(x, m, ldx, cols, qa, sa, blocks_pad, s);
+  else
+    aligned ? launch_quantize_tiles<false, true, T16>(x, m, ldx, cols, qa, sa, blocks_pad, s)
+            : launch_quantize_tiles<false, false, T16>(x, m, ldx, cols, qa, sa, blocks_pad, s);
 }
 
 hipError_t launch_quantize_tiled(const void *x, bool x_bf16, int64_t m,
@@ -1306,12 +1328,10 @@ hipError_t launch_quantize_tiled(const void *x, bool x_bf16, int64_t m,
                                  hipStream_t s) {
   const int64_t esz = x_bf16 ? 2 : 4;
   const bool aligned = ((uintptr_t)x % (4 * esz) == 0) && (ldx % 4 == 0);
-  if (x_bf16)
-    aligned ? launch_quantize_tiles<true, true>(x, m, ldx, cols, qa, sa, blocks_pad, t16, s)
-            : launch_quantize_tiles<true, false>(x, m, ldx, cols, qa, sa, blocks_pad, t16, s);
+  if (t16)
+    launch_quantize_layout<true>(x, x_bf16, aligned, m, ldx, cols, qa, sa, blocks_pad, s);
   else
-    aligned ? launch_quantize_tiles<false, true>(x, m, ldx, cols, qa, sa, blocks_pad, t16, s)
-            : launch_quantize_tiles<false, false>(x, m, ldx, cols, qa, sa, blocks_pad, t16, s);
+    launch_quantize_layout<false>(x, x_bf16, aligned, m, ldx, cols, qa, sa, blocks_pad, s);
   return hipGetLastError();
 }
 
