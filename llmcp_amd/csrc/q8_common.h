@@ -51,6 +51,27 @@ __host__ __device__ constexpr int seg_for(int64_t units) {
   return units == 18 ? 6 : (units == 8 ? 4 : 1);
 }
 
+// Buffer extent and scalar offset of one stage's DMA from a base address: the
+// whole 4 GiB that an unsigned offset reaches, or, for a stage that is not
+// there, nothing at offset 0.  A raw buffer load is in range while its lane
+// offset is below the extent less the scalar offset: with both zero no lane is,
+// whereas a scalar offset left on an empty extent would wrap that difference
+// round to a large one.  (On the device: kept in scalar registers.  As a plain
+// select the extent went through a vector register, and every buffer resource
+// made from it looked divergent.)
+struct DmaStage {
+  int32_t extent;
+  uint32_t offset;
+};
+__host__ __device__ inline DmaStage dma_stage(bool on, uint32_t offset) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const int32_t live = __builtin_amdgcn_readfirstlane(on ? -1 : 0);
+#else
+  const int32_t live = on ? -1 : 0;
+#endif
+  return {live, offset & (uint32_t)live};
+}
+
 // Unit and lane slot of block b for a compile-time S.
 template <int S>
 __host__ __device__ inline void locate(int64_t b, int64_t &unit, int &slot) {

@@ -103,16 +103,10 @@ struct Gemm16Shape {
   static_assert(LDS <= 160 * 1024, "LDS");
 };
 
-// The extent of the operands for a stage: the whole 4 GiB an unsigned
-// offset reaches, or nothing for one past the last (its loads return zeros
-// without touching memory, so no load is ever branched around).
-// readfirstlane keeps the value in a scalar register: as a plain select it
-// went through a vector register, and every buffer resource made from it
-// looked divergent.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void *p, bool on) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0,
-                                           __builtin_amdgcn_readfirstlane(on ? -1 : 0),
-                                           0x00020000);
+// The resource of a stage's operands (no load is ever branched around: one past
+// the last stage returns zeros without touching memory, dma_stage).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void *p, const DmaStage &st) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, st.extent, 0x00020000);
 }
 
 template <int N>
@@ -200,10 +194,12 @@ void gemm16_kernel(const Gemm16Args p) {
       }
       auto issue = [&](int t, int buf) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < Sh::DA; ++u)
+        for (int u = 0; u < Sh::DA; ++u) {
+          const DmaStage st = dma_stage(on[u] && t < stages, (uint32_t)t * ustep[u]);
           __builtin_amdgcn_raw_ptr_buffer_load_lds(
-              rsrc_of(base[u], on[u] && t < stages), (lds_void *)(smem + buf * Sh::ASZ + dst[u]),
-              16, voff[u], (uint32_t)t * ustep[u], 0, 0);
+              rsrc_of(base[u], st), (lds_void *)(smem + buf * Sh::ASZ + dst[u]), 16, voff[u],
+              st.offset, 0, 0);
+        }
       };
 #pragma unroll
       for (int i = 0; i < NA; ++i) issue(i, i);
@@ -264,18 +260,19 @@ void gemm16_kernel(const Gemm16Args p) {
         const uint32_t quarter = SEG == 1 ? 0u : (uint32_t)(s & 3);
         static_for<Sh::DB>([&](auto U) __attribute__((always_inline)) {
           constexpr int u = decltype(U)::value;
-          const auto r = rsrc_of(base[u], s < bstages);
+          const DmaStage st =
+              dma_stage(s < bstages, unit * kPassBytes + uoff[u] + quarter * uslot[u]);
+          const auto r = rsrc_of(base[u], st);
           const auto to = (lds_void *)(smem + Sh::BOFF + buf * Sh::BSZ + dst[u]);
-          const uint32_t off = unit * kPassBytes + uoff[u] + quarter * uslot[u];
           // up to 16 rows one workgroup alone reads these weights: non-temporal
           // (M = 16, N = 9216, K = 2560 13.9 -> 12.9 us from HBM; at 32 rows
           // 4 % less from HBM, 10 % more for weights that fit the 256 MB
           // cache behind it)
           constexpr int kNt = RT == 1 ? 2 : 0;
           if constexpr (u < Sh::DQ || SEG == 1)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, to, 16, voff[u], off, 0, kNt);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, to, 16, voff[u], st.offset, 0, kNt);
           else
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, to, 4, voff[u], off, 0, kNt);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, to, 4, voff[u], st.offset, 0, kNt);
         });
       };
 #pragma unroll

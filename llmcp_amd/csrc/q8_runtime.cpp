@@ -692,6 +692,16 @@ int llmcp_q8_test_ctx_gemm_splits(llmcp_q8_ctx *ctx, int32_t splits) {
   return LLMCP_Q8_OK;
 }
 
+// Test hook, declared in no header of the product (no counterpart in the
+// reference): extent and scalar offset that the GEMM's producer waves give
+// the DMA of a stage (dma_stage).
+void llmcp_q8_test_dma_stage(int32_t on, uint32_t offset, uint32_t *extent,
+                             uint32_t *scalar_offset) {
+  const DmaStage st = dma_stage(on != 0, offset);
+  *extent = (uint32_t)st.extent;
+  *scalar_offset = st.offset;
+}
+
 int32_t llmcp_q8_get_platform(llmcp_q8_ctx *ctx) {
   return ctx ? ctx->platform : -1;
 }
