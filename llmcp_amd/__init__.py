@@ -112,7 +112,7 @@ def lib():
         "llmcp_q8_abi_version": (I32, []),
         "llmcp_q8_test_ctx_rmsnorm_skew": (I, [P, I32]),
         "llmcp_q8_test_ctx_gemm_splits": (I, [P, I32]),
-        "llmcp_q8_test_dma_stage": (None, [I32, ctypes.c_uint32, P, P]),
+        "llmcp_q8_test_dma_stage": (None, [I32, I32, ctypes.c_uint32, P, P]),
         "llmcp_q8_set_accumulation": (I, [P, I32]),
         "llmcp_q8_microbench_bandwidth": (I, [P, I32, U64, I32, ctypes.POINTER(ctypes.c_double)]),
         "llmcp_q8_microbench_int8_mfma": (I, [P, I32, ctypes.POINTER(ctypes.c_double)]),

@@ -51,24 +51,24 @@ __host__ __device__ constexpr int seg_for(int64_t units) {
   return units == 18 ? 6 : (units == 8 ? 4 : 1);
 }
 
-// Buffer extent and scalar offset of one stage's DMA from a base address: the
-// whole 4 GiB that an unsigned offset reaches, or, for a stage that is not
-// there, nothing at offset 0.  A raw buffer load is in range while its lane
-// offset is below the extent less the scalar offset: with both zero no lane is,
-// whereas a scalar offset left on an empty extent would wrap that difference
-// round to a large one.  (On the device: kept in scalar registers.  As a plain
-// select the extent went through a vector register, and every buffer resource
-// made from it looked divergent.)
+// Buffer extent and scalar offset of the DMA of stage t of `stages`, `offset`
+// bytes from a base address: the whole 4 GiB that an unsigned offset reaches,
+// or, past the last stage, nothing at offset 0.  A raw buffer load is in range
+// while its lane offset is below the extent less the scalar offset: with both
+// zero no lane is, whereas a scalar offset left on an empty extent would wrap
+// that difference round to a large one.  (On the device the sign is taken
+// arithmetically, in scalar registers: as a select the extent goes through a
+// vector register, and every buffer resource made from it looks divergent.)
 struct DmaStage {
   int32_t extent;
   uint32_t offset;
 };
-__host__ __device__ inline DmaStage dma_stage(bool on, uint32_t offset) {
+__host__ __device__ inline DmaStage dma_stage(int32_t t, int32_t stages, uint32_t offset) {
+  int32_t left = t - stages;
 #ifdef __HIP_DEVICE_COMPILE__
-  const int32_t live = __builtin_amdgcn_readfirstlane(on ? -1 : 0);
-#else
-  const int32_t live = on ? -1 : 0;
+  asm("" : "+s"(left));  // or the compiler makes a compare and a select of it
 #endif
+  const int32_t live = left >> 31;  // -1 or 0
   return {live, offset & (uint32_t)live};
 }
 

@@ -169,7 +169,7 @@ void gemm16_kernel(const Gemm16Args p) {
       // A: per stage RT * 4 ops of values and one op of scales per two tiles
       uint32_t voff[Sh::DA], ustep[Sh::DA], dst[Sh::DA];
       const uint8_t *base[Sh::DA];
-      bool on[Sh::DA];
+      int32_t ends[Sh::DA];  // stages, none for a row tile past the last
 #pragma unroll
       for (int u = 0; u < Sh::DA; ++u) {
         int o = pw + u * Sh::P;
@@ -180,13 +180,13 @@ void gemm16_kernel(const Gemm16Args p) {
           // lanes 0-31 the eight blocks' scales of one tile, 32-63 of the next
           const int t0 = mg * RT + 2 * (o - RT * 4);
           const int tl = min(t0 + (lane >> 5), p.row_tiles - 1) - t0;
-          on[u] = t0 < p.row_tiles;
+          ends[u] = t0 < p.row_tiles ? stages : 0;
           ustep[u] = 512;
           base[u] = uniform_base(p.sa + (int64_t)t0 * nblk * 16);
           voff[u] = (uint32_t)max(tl, 0) * nblk * 64 + (lane & 31) * 16;
         } else {
           const int t0 = mg * RT + (o >> 2);
-          on[u] = t0 < p.row_tiles;
+          ends[u] = t0 < p.row_tiles ? stages : 0;
           ustep[u] = 4096;
           base[u] = uniform_base(p.qa + (int64_t)t0 * nblk * 512 + (o & 3) * 1024);
           voff[u] = lane * 16;
@@ -195,7 +195,7 @@ void gemm16_kernel(const Gemm16Args p) {
       auto issue = [&](int t, int buf) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < Sh::DA; ++u) {
-          const DmaStage st = dma_stage(on[u] && t < stages, (uint32_t)t * ustep[u]);
+          const DmaStage st = dma_stage(t, ends[u], (uint32_t)t * ustep[u]);
           __builtin_amdgcn_raw_ptr_buffer_load_lds(
               rsrc_of(base[u], st), (lds_void *)(smem + buf * Sh::ASZ + dst[u]), 16, voff[u],
               st.offset, 0, 0);
@@ -261,7 +261,7 @@ void gemm16_kernel(const Gemm16Args p) {
         static_for<Sh::DB>([&](auto U) __attribute__((always_inline)) {
           constexpr int u = decltype(U)::value;
           const DmaStage st =
-              dma_stage(s < bstages, unit * kPassBytes + uoff[u] + quarter * uslot[u]);
+              dma_stage(s, bstages, unit * kPassBytes + uoff[u] + quarter * uslot[u]);
           const auto r = rsrc_of(base[u], st);
           const auto to = (lds_void *)(smem + Sh::BOFF + buf * Sh::BSZ + dst[u]);
           // up to 16 rows one workgroup alone reads these weights: non-temporal

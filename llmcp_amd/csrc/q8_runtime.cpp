@@ -694,10 +694,10 @@ int llmcp_q8_test_ctx_gemm_splits(llmcp_q8_ctx *ctx, int32_t splits) {
 
 // Test hook, declared in no header of the product (no counterpart in the
 // reference): extent and scalar offset that the GEMM's producer waves give
-// the DMA of a stage (dma_stage).
-void llmcp_q8_test_dma_stage(int32_t on, uint32_t offset, uint32_t *extent,
+// the DMA of stage t of `stages` (dma_stage).
+void llmcp_q8_test_dma_stage(int32_t t, int32_t stages, uint32_t offset, uint32_t *extent,
                              uint32_t *scalar_offset) {
-  const DmaStage st = dma_stage(on != 0, offset);
+  const DmaStage st = dma_stage(t, stages, offset);
   *extent = (uint32_t)st.extent;
   *scalar_offset = st.offset;
 }

@@ -11,23 +11,25 @@ OFFSETS = [0, 512, 4096, 2176, 20 * 4096, 18 * 2176, 0x7FFFFFFF, 0x80000000, 0xF
 LANES = [0, 16, 1008, 4 * 5 * 2176, 0x7FFFFFF0, 0x80000000, 0xFFFFFFE0]
 
 
-def stage(q8, on, offset):
+def stage(q8, t, stages, offset):
     extent, scalar = ctypes.c_uint32(), ctypes.c_uint32()
-    q8.lib().llmcp_q8_test_dma_stage(on, offset, ctypes.byref(extent), ctypes.byref(scalar))
+    q8.lib().llmcp_q8_test_dma_stage(t, stages, offset, ctypes.byref(extent), ctypes.byref(scalar))
     return extent.value, scalar.value
 
 
 @pytest.mark.parametrize("offset", OFFSETS)
-def test_stage_past_the_last_reads_nothing(q8, offset):
+@pytest.mark.parametrize("t,stages", [(0, 0), (3, 0), (10, 10), (13, 10), (4 * 10**6, 10)])
+def test_stage_past_the_last_reads_nothing(q8, t, stages, offset):
     """A raw buffer load is in range where its lane offset is below extent -
     scalar offset (mod 2^32); a stage that is not there must have no lane in
     range, whether the scalar offset takes part in the check or not."""
-    extent, scalar = stage(q8, 0, offset)
+    extent, scalar = stage(q8, t, stages, offset)
     for lane in LANES:
         assert not lane < (extent - scalar) % 2**32, (offset, lane)
         assert not lane < extent and not lane + scalar < extent, (offset, lane)
 
 
 @pytest.mark.parametrize("offset", OFFSETS)
-def test_stage_that_is_there_keeps_its_offset(q8, offset):
-    assert stage(q8, 1, offset) == (0xFFFFFFFF, offset)
+@pytest.mark.parametrize("t,stages", [(0, 1), (9, 10), (0, 4 * 10**6)])
+def test_stage_that_is_there_keeps_its_offset(q8, t, stages, offset):
+    assert stage(q8, t, stages, offset) == (0xFFFFFFFF, offset)
