@@ -107,9 +107,8 @@ enum llmcp_q8_platform {
  *                  reference within 1e-5 relative or 1e-4 absolute (bf16
  *                  outputs within one bf16 step); the same inputs give the
  *                  same bits on every call.  One-row calls, the lm_head
- *                  (logits and argmax), shapes that fill the GPU and shapes
- *                  that the GEMM on 16 x 16 tiles serves at least as fast in
- *                  the serial order run as in EXACT.  Needs workspace for the partial sums, grown on
+ *                  (logits and argmax) and shapes that fill the GPU run as
+ *                  in EXACT.  Needs workspace for the partial sums, grown on
  *                  first use like the prefill scratch. */
 enum llmcp_q8_accumulation {
   LLMCP_Q8_ACCUM_EXACT = 0,

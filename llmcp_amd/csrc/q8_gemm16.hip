@@ -573,10 +573,10 @@ hipError_t launch16_f(Gemm16Args &a, const Gemm16Launch &l, int32_t rts, const S
 // 32 / 64 15.4 / 15.7 / 15.8 -> 12.9 / 15.8 / 18.2 (the last two not taken);
 // its SwiGLU M = 16 / 32 29.6 / 30.3 -> 17.5 / 23.3; N = 2560, K = 9216 / 4096
 // M = 333 104.9 / 45.4 -> 73.6 / 38.1.
-// Where K may be split (split_k) a second round loses to the splits (N =
-// 2560, K = 9216, M = 512: 73 us), one round does not (M = 256: 50).
-bool gemm16_takes(int64_t m, const int64_t *rows, int count, int64_t cols, bool dual,
-                  bool split_k) {
+// SPLIT_K is no choice to make here: what splits K must depend on the one
+// linear, whatever else shares its launch, so the caller keeps linears that
+// split on launch_gemm.
+bool gemm16_takes(int64_t m, const int64_t *rows, int count, int64_t cols, bool dual) {
   if (m <= 1) return false;
   const int64_t cus = cu_count(), units = passes_for(cols), rts = (m + 15) / 16;
   const double blocks = (double)units * kPassBlocks;
@@ -591,9 +591,7 @@ bool gemm16_takes(int64_t m, const int64_t *rows, int count, int64_t cols, bool 
     old_us += us * (dual ? 2 : 1);
   }
   const Shape16 sh = shape16(rts, tiles, seg_for(units), dual);
-  const int64_t rounds = rounds16(sh, rts, tiles);
-  if (split_k && rounds > 1) return false;
-  return 5.0 + (double)rounds * sh.per_block * blocks < old_us;
+  return 5.0 + (double)rounds16(sh, rts, tiles) * sh.per_block * blocks < old_us;
 }
 
 hipError_t launch_gemm16(const Gemm16Launch &l, hipStream_t s) {

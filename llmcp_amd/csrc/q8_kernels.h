@@ -162,10 +162,9 @@ struct Gemm16Launch {
 };
 hipError_t launch_gemm16(const Gemm16Launch &l, hipStream_t s);
 // Whether m rows go to launch_gemm16, for `count` weights [rows[i] x cols] in
-// one launch (dual: one SwiGLU pair), rather than to launch_gemm for each.
-// split_k: launch_gemm could split K.
-bool gemm16_takes(int64_t m, const int64_t *rows, int count, int64_t cols, bool dual,
-                  bool split_k);
+// one launch (dual: one SwiGLU pair), rather than to launch_gemm for each,
+// unsplit.
+bool gemm16_takes(int64_t m, const int64_t *rows, int count, int64_t cols, bool dual);
 
 // K splits for a multi-row linear of [m x cols] by [rows x cols] when
 // splitting is allowed: `forced` > 0 (clamped to the pass count), else the

@@ -1113,20 +1113,27 @@ static int gemm_quantize(llmcp_q8_ctx *ctx, const Rows &in, const Tensor *w,
   return LLMCP_Q8_OK;
 }
 
+// K splits of m rows of w: one in EXACT mode, for the lm_head (`exact`) and for
+// shapes that do not gain from more.  It depends on this linear alone, so that
+// a call sums in one order whether it comes by itself or in a group.
+static int32_t splits_for(llmcp_q8_ctx *ctx, int64_t m, const Tensor *w, bool exact) {
+  if (exact || ctx->accumulation != LLMCP_Q8_ACCUM_SPLIT_K || w->rows % 4 != 0) return 1;
+  return gemm_splits_for(m, w->rows, w->cols, ctx->test_splits);
+}
+
 // Whether these rows take the 16 x 16-tile GEMM, for `count` weights in one
-// launch (outputs of one element type).  It sums in the serial block order,
-// so it serves both accumulation modes; only a forced split count (a test
-// hook) goes past it.
+// launch (outputs of one element type).  It sums in the serial block order:
+// a linear that splits K goes past it, and so does any with a forced split
+// count (a test hook).
 static bool gemm16_for(llmcp_q8_ctx *ctx, int64_t m, int32_t count, const Tensor *const *w,
-                       const Rows *outs, bool dual = false) {
-  const bool split_k = ctx->accumulation == LLMCP_Q8_ACCUM_SPLIT_K;
-  if (split_k && ctx->test_splits > 0) return false;
+                       const Rows *outs, bool dual = false, bool exact = false) {
+  if (!exact && ctx->accumulation == LLMCP_Q8_ACCUM_SPLIT_K && ctx->test_splits > 0) return false;
   int64_t rows[kMaxGroup];
   for (int32_t i = 0; i < count; ++i) {
-    if (outs[i].bf16 != outs[0].bf16) return false;
+    if (outs[i].bf16 != outs[0].bf16 || splits_for(ctx, m, w[i], exact) > 1) return false;
     rows[i] = w[i]->rows;
   }
-  return gemm16_takes(m, rows, count, w[0]->cols, dual, split_k);
+  return gemm16_takes(m, rows, count, w[0]->cols, dual);
 }
 
 // The 16 x 16-tile GEMM of the quantized rows: `count` weights in one
@@ -1194,16 +1201,13 @@ static int gemm_launch(llmcp_q8_ctx *ctx, const Workspace &ws, int64_t m,
     g.add = residual->data;
     g.ldr = residual->ld;
   }
-  if (!exact && ctx->accumulation == LLMCP_Q8_ACCUM_SPLIT_K && !ws.fixed &&
-      w->rows % 4 == 0) {
-    const int32_t splits = gemm_splits_for(m, w->rows, w->cols, ctx->test_splits);
-    if (splits > 1) {
-      const uint64_t bytes = (uint64_t)splits * (uint64_t)m * (uint64_t)w->rows * 4u;
-      int rc = grow(ctx, ctx->part, ctx->part_bytes, bytes, "split-K partial sums");
-      if (rc) return rc;
-      g.splits = splits;
-      g.part = ctx->part;
-    }
+  const int32_t splits = ws.fixed ? 1 : splits_for(ctx, m, w, exact);
+  if (splits > 1) {
+    const uint64_t bytes = (uint64_t)splits * (uint64_t)m * (uint64_t)w->rows * 4u;
+    int rc = grow(ctx, ctx->part, ctx->part_bytes, bytes, "split-K partial sums");
+    if (rc) return rc;
+    g.splits = splits;
+    g.part = ctx->part;
   }
   hipError_t e = launch_gemm(g, ctx->stream);
   if (e != hipSuccess) return hip_fail(e, "gemm launch");
@@ -1214,7 +1218,7 @@ static int gemm_common(llmcp_q8_ctx *ctx, const Rows &in, const Tensor *w,
                        const Rows &out, int activation,
                        const Workspace *fixed = nullptr, bool exact = false) {
   Workspace ws = fixed ? *fixed : ctx_workspace(ctx);
-  const bool t16 = gemm16_for(ctx, in.rows, 1, &w, &out);
+  const bool t16 = gemm16_for(ctx, in.rows, 1, &w, &out, false, exact);
   int rc = gemm_quantize(ctx, in, w, ws, t16);
   if (rc) return rc;
   if (t16) return gemm16_launch(ctx, ws, in.rows, &w, nullptr, &out, &activation, 1);
