@@ -1496,6 +1496,24 @@ static int rmsnorm_group_impl(llmcp_q8_ctx *ctx, const Rows &in, const NormWeigh
   return linear_group_run(ctx, normed, count, w, outs, acts, true);
 }
 
+// Where the gate's rows of a SwiGLU into `out` go when gate and up are two
+// GEMMs.  f32: straight into the output, and the up GEMM multiplies it in
+// place.  bf16: to f32 scratch, and the multiply rounds both factors to bf16
+// first.  The scratch grows whichever GEMM these rows take: the choice goes
+// back and forth with M, and a program that has run more rows may capture fewer
+// without an allocation.
+static int swiglu_gate_rows(llmcp_q8_ctx *ctx, int64_t m, const Rows &out, Rows &g) {
+  g = out;
+  if (!out.bf16) return LLMCP_Q8_OK;
+  int rc = grow(ctx, ctx->up, ctx->up_bytes, (uint64_t)(m * out.cols) * 4,
+                "prefill SwiGLU scratch");
+  if (rc) return rc;
+  g.data = ctx->up;
+  g.bf16 = false;
+  g.ld = out.cols;
+  return LLMCP_Q8_OK;
+}
+
 static int swiglu_impl(llmcp_q8_ctx *ctx, const Rows &in,
                        const llmcp_memref_i8_1d *w_gate,
                        const llmcp_memref_i8_1d *w_up, const Rows &out,
@@ -1512,6 +1530,8 @@ static int swiglu_impl(llmcp_q8_ctx *ctx, const Rows &in,
   if (m == 0) return LLMCP_Q8_OK;
   if ((rc = set_device(ctx))) return rc;
   if (m == 1) return gemv_common(ctx, in, wg, wu, out, LLMCP_Q8_ACT_NONE, nullptr);
+  Rows g;
+  if ((rc = swiglu_gate_rows(ctx, m, out, g))) return rc;
   if (gemm16_for(ctx, m, 1, &wg, &out, true)) {
     Workspace ws = ctx_workspace(ctx);
     if ((rc = gemm_operands_fit(wu, m)) || (rc = gemm_quantize(ctx, in, wg, ws, true)))
@@ -1520,19 +1540,7 @@ static int swiglu_impl(llmcp_q8_ctx *ctx, const Rows &in,
   }
   // Several rows: the input quantized once; the gate GEMM with SiLU, then the up
   // GEMM whose epilogue does the multiply (MulOpLowering,
-  // LowerToLinalg.cpp:377-393) with the gate's output.  f32: the gate goes
-  // straight into the output and the up GEMM multiplies it in place.  bf16:
-  // the gate goes to f32 scratch and the multiply rounds both factors to
-  // bf16 first.
-  Rows g = out;
-  if (out.bf16) {
-    rc = grow(ctx, ctx->up, ctx->up_bytes, (uint64_t)(m * wg->rows) * 4,
-              "prefill SwiGLU scratch");
-    if (rc) return rc;
-    g.data = ctx->up;
-    g.bf16 = false;
-    g.ld = wg->rows;
-  }
+  // LowerToLinalg.cpp:377-393) with the gate's output.
   Workspace ws = ctx_workspace(ctx);
   if ((rc = gemm_quantize(ctx, in, wg, ws, false))) return rc;
   if ((rc = gemm_launch(ctx, ws, m, wg, g, LLMCP_Q8_ACT_SILU, nullptr, 0)))
@@ -1623,20 +1631,13 @@ static int mlp_impl(llmcp_q8_ctx *ctx, const Rows &in,
       h.cols = h.ld = f;
       h.bf16 = out.bf16;
     }
+    Rows g;
+    if ((rc = swiglu_gate_rows(ctx, m, h, g))) return rc;
     if (gemm16_for(ctx, m, 1, &wg, &h, true)) {
       Workspace ws = ctx_workspace(ctx);
       if ((rc = gemm_quantize(ctx, in, wg, ws, true))) return rc;
       if ((rc = gemm16_launch(ctx, ws, m, &wg, wu, &h, nullptr, 1))) return rc;
       return gemm_common(ctx, h, wd, out, LLMCP_Q8_ACT_NONE);
-    }
-    Rows g = h;  // the gate's output: h itself (f32) or f32 scratch (bf16)
-    if (h.bf16) {
-      if ((rc = grow(ctx, ctx->up, ctx->up_bytes, (uint64_t)(m * f) * 4,
-                     "prefill SwiGLU scratch")))
-        return rc;
-      g.data = ctx->up;
-      g.bf16 = false;
-      g.ld = f;
     }
     Workspace ws = ctx_workspace(ctx);
     if ((rc = gemm_quantize(ctx, in, wg, ws, false))) return rc;

@@ -61,3 +61,42 @@ def test_split_shapes_run_in_their_splits(ctx, oracle, m, n, k, splits):
     finally:
         ctx.set_accumulation("exact")
         ctx.release(t)
+
+
+@pytest.mark.parametrize("entry", ["swiglu", "mlp"])
+def test_warm_up_with_more_rows_prepares_fewer(q8, oracle, entry):
+    """A call of more rows prepares the scratch of one with fewer, also where
+    the two run on different GEMMs: H = 1024, F = 4352 in bf16 takes the 16 x
+    16 tiles at 100 rows and the 64 x 64 ones, which need a buffer for the
+    gate, at 40.  Each replay equals the eager result."""
+    h, f, rng = 1024, 4352, np.random.default_rng(3)
+    with q8.Context(0) as c:
+        ts = [c.upload_p4(weights(oracle, rng, n, k), n, k) for n, k in ((f, h), (f, h), (h, f))]
+        x = oracle.f32_to_bf16_bits(rng.standard_normal((100, h)).astype(np.float32))
+        xd, hd, yd = c.to_device(x), c.alloc(100 * f * 2), c.alloc(100 * h * 2)
+
+        def call(m):
+            if entry == "swiglu":
+                c.swiglu(xd, ts[0], ts[1], hd, m, mode="prefill", dtype="bf16")
+            else:
+                c.mlp(xd, ts[0], ts[1], ts[2], yd, h=hd, m=m, mode="prefill", dtype="bf16")
+
+        def result():
+            return (c.to_host(hd, (40, f), np.uint16) if entry == "swiglu"
+                    else c.to_host(yd, (40, h), np.uint16))
+
+        call(100)
+        c.sync()
+        c.graph_begin()
+        call(40)
+        graph = c.graph_end()
+        replays = []
+        for _ in range(3):
+            c.graph_launch(graph)
+            c.sync()
+            replays.append(result())
+        call(40)
+        c.sync()
+        for got in replays:
+            assert np.array_equal(got, result())
+        c.graph_destroy(graph)
