@@ -112,6 +112,7 @@ def lib():
         "llmcp_q8_abi_version": (I32, []),
         "llmcp_q8_test_ctx_rmsnorm_skew": (I, [P, I32]),
         "llmcp_q8_test_ctx_gemm_splits": (I, [P, I32]),
+        "llmcp_q8_test_gemm_plan": (I32, [I64, P, I32, I64, I32, P, P, P, P]),
         "llmcp_q8_test_dma_stage": (None, [I32, I32, ctypes.c_uint32, P, P]),
         "llmcp_q8_set_accumulation": (I, [P, I32]),
         "llmcp_q8_microbench_bandwidth": (I, [P, I32, U64, I32, ctypes.POINTER(ctypes.c_double)]),
@@ -611,6 +612,18 @@ class Context:
 
     def graph_destroy(self, g):
         check(lib().llmcp_q8_graph_destroy(g))
+
+
+def gemm_plan(m, rows, cols, dual=False):
+    """The kernel of m input rows against weights [rows[i] x cols] in one call
+    (dual: a SwiGLU pair), a test hook: (S, row tiles, column tiles) of the
+    GEMM on 16 x 16 tiles or None for the other GEMM, and the K splits of the
+    first weight by itself in split_k mode."""
+    n = np.asarray(rows, np.int64)
+    out = np.zeros(4, np.int32)
+    at = [out.ctypes.data + 4 * i for i in range(4)]
+    taken = lib().llmcp_q8_test_gemm_plan(m, n.ctypes.data, len(n), cols, int(dual), *at)
+    return (tuple(int(v) for v in out[:3]) if taken else None), int(out[3])
 
 
 def pack_p4_host(w):

@@ -594,6 +594,16 @@ bool gemm16_takes(int64_t m, const int64_t *rows, int count, int64_t cols, bool 
   return 5.0 + (double)rounds16(sh, rts, tiles) * sh.per_block * blocks < old_us;
 }
 
+void gemm16_instance(int64_t m, const int64_t *rows, int count, int64_t cols, bool dual,
+                     int32_t *seg, int32_t *row_tiles, int32_t *col_tiles) {
+  int64_t tiles = 0;
+  for (int i = 0; i < count; ++i) tiles += (rows[i] + 15) / 16;
+  *seg = seg_for(passes_for(cols));
+  const Shape16 sh = shape16((m + 15) / 16, tiles, *seg, dual);
+  *row_tiles = sh.rt;
+  *col_tiles = sh.cn;
+}
+
 hipError_t launch_gemm16(const Gemm16Launch &l, hipStream_t s) {
   Gemm16Args a = {};
   a.qa = l.qa;

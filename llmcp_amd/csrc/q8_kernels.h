@@ -165,6 +165,10 @@ hipError_t launch_gemm16(const Gemm16Launch &l, hipStream_t s);
 // one launch (dual: one SwiGLU pair), rather than to launch_gemm for each,
 // unsplit.
 bool gemm16_takes(int64_t m, const int64_t *rows, int count, int64_t cols, bool dual);
+// The kernel that launch_gemm16 runs for them: the weights' S (seg_for) and
+// the workgroup's row and column tiles.
+void gemm16_instance(int64_t m, const int64_t *rows, int count, int64_t cols, bool dual,
+                     int32_t *seg, int32_t *row_tiles, int32_t *col_tiles);
 
 // K splits for a multi-row linear of [m x cols] by [rows x cols] when
 // splitting is allowed: `forced` > 0 (clamped to the pass count), else the

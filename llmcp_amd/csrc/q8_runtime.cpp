@@ -702,6 +702,19 @@ void llmcp_q8_test_dma_stage(int32_t t, int32_t stages, uint32_t offset, uint32_
   *scalar_offset = st.offset;
 }
 
+// Test hook, declared in no header of the product (no counterpart in the
+// reference): which kernel m rows of `count` weights [rows[i] x cols] (dual:
+// of one SwiGLU pair) run on.  Returns 1 for the GEMM on 16 x 16 tiles (then
+// its instance), 0 for the other; `splits`: the K splits of weight 0 by
+// itself in SPLIT_K mode.
+int32_t llmcp_q8_test_gemm_plan(int64_t m, const int64_t *rows, int32_t count, int64_t cols,
+                                int32_t dual, int32_t *seg, int32_t *row_tiles,
+                                int32_t *col_tiles, int32_t *splits) {
+  gemm16_instance(m, rows, count, cols, dual != 0, seg, row_tiles, col_tiles);
+  *splits = gemm_splits_for(m, rows[0], cols, 0);
+  return gemm16_takes(m, rows, count, cols, dual != 0) ? 1 : 0;
+}
+
 int32_t llmcp_q8_get_platform(llmcp_q8_ctx *ctx) {
   return ctx ? ctx->platform : -1;
 }

@@ -33,3 +33,11 @@ def test_stage_past_the_last_reads_nothing(q8, t, stages, offset):
 @pytest.mark.parametrize("t,stages", [(0, 1), (9, 10), (0, 4 * 10**6)])
 def test_stage_that_is_there_keeps_its_offset(q8, t, stages, offset):
     assert stage(q8, t, stages, offset) == (0xFFFFFFFF, offset)
+
+
+# the shapes that tests/test_gpu_split.py names as splitting by their own choice
+@pytest.mark.parametrize("m,n,k", [(2, 136, 1024), (33, 520, 2560), (97, 2560, 9216),
+                                   (40, 264, 4096), (200, 2560, 2560), (48, 1024, 2560),
+                                   (32, 2560, 2560), (16, 2560, 9216), (64, 256, 2560)])
+def test_shapes_of_the_split_tests_split(q8, m, n, k):
+    assert q8.gemm_plan(m, [n], k)[1] > 1
