@@ -283,9 +283,10 @@ def bench_gemm(ctx, m, n=9216, k=2560, iters=30):
 
 def bench_split_k(ctx, n=2560, k=9216, ms=(64, 256)):
     """The SPLIT_K accumulation mode (opt-in, within the north-star
-    tolerance) against EXACT on the down projection's shape at few rows,
-    where K = 9216 runs 72 serial stages per tile: op times of the same
-    calls in both modes (the count of splits is the library's choice)."""
+    tolerance) against EXACT on the down projection's shape at few rows:
+    op times of the same calls in both modes (the count of splits is the
+    library's choice; EXACT runs one serial chain over K = 9216 per output,
+    on 16 x 16 tiles at these rows)."""
     out = {}
     for m in ms:
         fig = {}

@@ -949,8 +949,11 @@ int32_t gemm_splits_for(int64_t m, int64_t rows, int64_t cols, int32_t forced) {
   if (forced > 0) return std::min(forced, passes);
   // As many splits as keep tiles x splits within one workgroup per CU, and
   // at most max(3, passes / 3) (three passes per split where K has nine or
-  // more).  Measured op time (quantizer, GEMM, reduction) against EXACT,
-  // splits in brackets:
+  // more).  Measured op time (quantizer, GEMM, reduction) against one split
+  // (EXACT itself may run on 16 x 16 tiles, q8_gemm16.hip, and is then often the
+  // faster: N = 2560, K = 9216 M = 64 / 256 / 512 24.0 / 43.3 / 79.0 against 26.4 /
+  // 49.5 / 78.0 split; N = 512, K = 16384, M = 16 22.7 against 19.4), splits in
+  // brackets:
   //   N = 2560, K = 9216: M = 64 65.9 -> 26.9 us (6); M = 128 109.8 -> 37.6
   //     (6; 9 splits 50.1); M = 256 109.2 -> 48.7 (4; 6 splits 61.6);
   //     M = 512 107.7 -> 72.8 (2; 3 splits 92.2); M = 1024 127.8, every

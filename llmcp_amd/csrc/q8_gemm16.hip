@@ -82,7 +82,7 @@ struct Gemm16Shape {
   // eight A stages (S = 6: nine).  The SwiGLU pair of one row tile leaves
   // room for three workgroups per CU instead: at N = 9216 that puts all 576
   // in flight at once (19.3 us against 25.9 with four pairs of tiles in 144
-  // deep workgroups, M = 16, K = 2560; 17.7 with the non-temporal loads).
+  // deep workgroups, M = 16, K = 2560; 16.8 with the non-temporal loads).
   static constexpr int BUDGET = (DUAL && RT == 1 ? 53 : 160) * 1024;
   static constexpr bool fits(int na, int nb) { return na * ASZ + nb * BSZ <= BUDGET; }
   static constexpr int NA = SEG != 6 && (fits(4, 4) || (!fits(3, 3) && fits(4, 2))) ? 4 : 3;
@@ -494,11 +494,11 @@ hipError_t launch16(Gemm16Args &a, const Gemm16Launch &l, int32_t row_tiles16, h
 // first (a column tile's weights are fetched once per RT rows), then the
 // fewest columns that put every workgroup on a CU of its own.  `per_block`
 // is a round's time per block of K, in us, fitted with 5 us of launch, fill
-// and input quantization to op times at N = 1000 .. 9216 (f32, aarch64):
-// (1, 1) 9.6 us at K = 2560, 18.6 at 9216; (1, 4) 12.9 at N = 9216, K =
-// 2560; (4, 1) 10.9 / 14.0 / 23.9 at K = 2560 / 4096 / 9216; (4, 2) 13.7 /
-// - / 33; (4, 3) 16.7 / 23.2 / 43.8; SwiGLU (1, 1) 12.4 at N = 2560, 17.5 at
-// 9216, (2, 3) 23.2, (4, 1) 15.2 .. 16.7 at K = 2560.
+// and input quantization to op times within 2 us (f32, aarch64): (1, 1) 8.0 ..
+// 8.4 us at K = 2560, 19.0 at 9216; (1, 4) 12.5 at N = 9216, K = 2560; (4, 1)
+// 10.9 / 13.7 / 24.0 at K = 2560 / 4096 / 9216; (4, 2) 13.4 / - / 31.8; (4, 3)
+// 16.0 / 21.9 / 43.3; SwiGLU (1, 1) 10.9 at N = 2560, 16.8 at 9216, (2, 3)
+// 23.5, (4, 1) 13.8 .. 14.9 at K = 2560.
 struct Shape16 {
   int rt, cn;
   double per_block;
@@ -562,17 +562,18 @@ hipError_t launch16_f(Gemm16Args &a, const Gemm16Launch &l, int32_t rts, const S
 }  // namespace
 
 // The cheaper of the two GEMMs by the fitted op times.  launch_gemm, exact:
-// up to 64 rows 1 + 0.18 us per block for one 64 x 64 workgroup per CU (14.2
-// .. 15.9 us at K = 2560, 26 at 4096, 54 at 9216) and 1 + 0.28 for each two
-// (178 us at N = 248320, K = 2560, M = 32), above 0.33 us per
-// block and round of 128 x 96 ones (25 .. 30 us at K = 2560, 45 at 4096, 105
-// at 9216), for each weight apart.  Op times launch_gemm -> launch_gemm16:
-// N = 2560, K = 9216 M = 2 / 64 / 256 / 512 53.8 / 56.2 / 105.6 / 105.0 ->
-// 18.9 / 23.9 / 43.8 / 81.1; N = 2560, K = 2560 M = 64 / 256 / 320 14.2 /
-// 26.0 / 26.2 -> 10.9 / 16.7 / 27.1 (not taken); N = 9216, K = 2560 M = 16 /
-// 32 / 64 15.4 / 15.7 / 15.8 -> 12.9 / 15.8 / 18.2 (the last two not taken);
-// its SwiGLU M = 16 / 32 29.6 / 30.3 -> 17.5 / 23.3; N = 2560, K = 9216 / 4096
-// M = 333 104.9 / 45.4 -> 73.6 / 38.1.
+// up to 64 rows 1 + 0.18 us per block for one 64 x 64 workgroup per CU (13.9
+// .. 15.8 us at K = 2560, 27 at 4096, 53 .. 56 at 9216) and 1 + 0.28 for each
+// two (188 us at N = 248320, K = 2560, M = 32), above 0.33 us per block and
+// round of 128 x 96 ones (26 .. 30 us at K = 2560, 45 at 4096, 105 at 9216),
+// for each weight apart.  Op times launch_gemm -> launch_gemm16:
+// N = 2560, K = 9216 M = 2 / 64 / 256 / 512 53.1 / 55.8 / 105.5 / 106.8 ->
+// 18.5 / 24.0 / 42.9 / 76.9; N = 2560, K = 2560 M = 64 / 256 / 320 13.9 /
+// 26.1 / 26.6 -> 10.9 / 16.0 / 25.5 (the last not taken); N = 9216, K = 2560
+// M = 16 / 32 / 64 15.0 / 15.3 / 15.8 -> 11.9 / 14.6 / 16.7 (the last two not
+// taken); its SwiGLU M = 16 / 32 / 64 29.5 / 30.2 / 31.0 -> 16.7 / 23.5 / 36.0
+// (the last not taken); N = 2560, K = 9216 / 4096, M = 333 106.2 / 46.1 -> 69.2 /
+// 36.5.
 // SPLIT_K is no choice to make here: what splits K must depend on the one
 // linear, whatever else shares its launch, so the caller keeps linears that
 // split on launch_gemm.

@@ -957,7 +957,7 @@ __global__ __launch_bounds__(512) void gated_rmsnorm_kernel(
 // floats, so that sixteen lanes' 16 B reads fall in different banks).  A fold
 // by a whole wave takes a wave slot for 128 dependent additions per group:
 // bound by rounds of workgroups, 10656 groups of 128 (333 rows of 4096, bf16)
-// took 11.2 us so, 6.8 here (26 MB: 3.9 TB/s).
+// took 11.2 us so, 6.8 here (8.2 MB, 1.2 TB/s: the additions bound it still).
 constexpr int kGatedManyG = 256;
 constexpr int kGatedMany = 16;                     // groups per workgroup
 constexpr int kGatedManySlots = kGatedManyG * kGatedMany / 4 / 256;  // float4s per lane
